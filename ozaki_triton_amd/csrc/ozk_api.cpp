@@ -91,20 +91,25 @@ ozk::SplitParams make_split_params(const void *X, int64_t batch, int64_t rows, i
     p.cs_b = cs[0];
     p.cs_l = cs[1];
     p.cs_r = cs[2];
+    p.Kp = K;
+    p.cols = 0;
+    p.x_code = 0;
     p.resid = nullptr;
     p.fail_out = nullptr;
     return p;
 }
 
 // Bytes of the packed copy of one slice operand, or 0 when it is already in
-// the layout the MFMA kernel reads: K-contiguous, 16-byte aligned rows/planes.
+// the layout the MFMA kernel reads: K-contiguous, 16-byte aligned rows/planes,
+// whole 16-byte pieces of K (or rows zero-padded to them).
 int64_t pack_bytes(const void *ptr, const int64_t s[4], int64_t batch, int L, int64_t rows,
-                   int64_t K, int es, bool is_b) {
+                   int64_t K, int es, bool is_b, bool zero_padded = false) {
     // a_strides = (b, l, m, k); b_strides = (b, l, k, n)
     const int64_t sk = is_b ? s[2] : s[3];
     const int64_t sr = is_b ? s[3] : s[2];
     const bool ok = sk == 1 && ((uintptr_t)ptr % 16) == 0 && (sr * es) % 16 == 0 &&
-                    (s[1] * es) % 16 == 0 && (s[0] * es) % 16 == 0 && (K * es) % 16 == 0;
+                    (s[1] * es) % 16 == 0 && (s[0] * es) % 16 == 0 &&
+                    (zero_padded || (K * es) % 16 == 0);
     if (ok || rows == 0 || K == 0 || L == 0) return 0;
     const int64_t kp = round_up(K * es, 16) / es;
     return round_up(batch * L * rows * kp * es, 256);
@@ -235,7 +240,8 @@ static int cross_gemm_impl(const void *A_slices, const int64_t a_strides[4], con
                    const int64_t sb_strides[3], int64_t batch, int64_t M, int64_t N, int64_t K,
                    int num_splits, int slice_dtype, int pairs, void *C, int out_dtype,
                    const int64_t c_strides[3], void *workspace, size_t workspace_bytes,
-                   void *stream, const uint32_t *const split_fail[2] = nullptr) {
+                   void *stream, const uint32_t *const split_fail[2] = nullptr,
+                   bool zero_padded = false) {
     if (!a_strides || !b_strides || !sa_strides || !sb_strides || !c_strides)
         return OZK_ERR_NULL;
     if (!is_slice_dtype(slice_dtype) || !is_input_dtype(out_dtype)) return OZK_ERR_DTYPE;
@@ -276,8 +282,10 @@ static int cross_gemm_impl(const void *A_slices, const int64_t a_strides[4], con
     if (!A_slices || !B_slices || !A_scales || !B_scales) return OZK_ERR_NULL;
 
     const int es = slice_size(slice_dtype);
-    const int64_t abytes = pack_bytes(A_slices, a_strides, batch, num_splits, M, K, es, false);
-    const int64_t bbytes = pack_bytes(B_slices, b_strides, batch, num_splits, N, K, es, true);
+    const int64_t abytes =
+        pack_bytes(A_slices, a_strides, batch, num_splits, M, K, es, false, zero_padded);
+    const int64_t bbytes =
+        pack_bytes(B_slices, b_strides, batch, num_splits, N, K, es, true, zero_padded);
     if (abytes + bbytes > 0 && (!workspace || workspace_bytes < (size_t)(abytes + bbytes) ||
                                 (uintptr_t)workspace % 16 != 0))
         return OZK_ERR_WORKSPACE;
@@ -370,9 +378,11 @@ int ozk_cross_gemm_pairs(const void *A_slices, const int64_t a_strides[4], const
 // alpha, the split of B through its transposed view and of A, and the
 // cross-GEMM, enqueued on one stream from one call; everything temporary
 // (slices, scales, scratch) lives in the caller's workspace:
-//   [A slices][A scales][B slices][B scales][split scratch][pack scratch],
-// each region 256-byte aligned.  A broadcast operand (batch stride 0) is split
-// once.
+//   [A slices][A scales][B slices][B scales][split scratch][split-K buffers],
+// each region 256-byte aligned.  Slice rows are padded with zeros to whole
+// 16-byte pieces, so that the cross-GEMM reads them in place whatever K is (a
+// packed copy of both operands took 121 of 990 us at 2049 x 3000 x 2047, 4
+// int8 slices).  A broadcast operand (batch stride 0) is split once.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -381,9 +391,10 @@ size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 struct MatmulLayout {
     int alpha;
     int64_t bA, bB;                                 // split batches (1 when broadcast)
-    size_t a_sl, a_sc, b_sl, b_sc, scratch, pack;   // byte offsets
+    int64_t kp;                                     // elements of a padded slice row
+    size_t a_sl, a_sc, b_sl, b_sc, scratch, sk;     // byte offsets
     size_t scratch_bytes;                           // split scratch reserved
-    size_t splitk;                                  // cross-GEMM split-K buffers (after pack)
+    size_t splitk;                                  // cross-GEMM split-K buffers, at sk
     size_t total;
     int64_t bt_strides[3];                          // B^T view of B
     int64_t ga[4], gb[4], gsa[3], gsb[3];           // cross-GEMM strides of the slices
@@ -425,11 +436,12 @@ int matmul_layout(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
     o->bt_strides[1] = bs[2];
     o->bt_strides[2] = bs[1];
     const int64_t ss = slice_size(sd);
-    const int64_t asl[4] = {L * M * K, M * K, K, 1}, bsl[4] = {L * N * K, N * K, K, 1};
+    const int64_t kp = o->kp = round_up(K * ss, 16) / ss;
+    const int64_t asl[4] = {L * M * kp, M * kp, kp, 1}, bsl[4] = {L * N * kp, N * kp, kp, 1};
     size_t off = 0;
-    o->a_sl = off; off = align256(off + (size_t)(o->bA * L * M * K * ss));
+    o->a_sl = off; off = align256(off + (size_t)(o->bA * L * M * kp * ss));
     o->a_sc = off; off = align256(off + (size_t)(o->bA * L * M * 4));
-    o->b_sl = off; off = align256(off + (size_t)(o->bB * L * N * K * ss));
+    o->b_sl = off; off = align256(off + (size_t)(o->bB * L * N * kp * ss));
     o->b_sc = off; off = align256(off + (size_t)(o->bB * L * N * 4));
     // the split scratch is sized for 256-byte aligned operands; plan_split
     // keeps the plan of any other pointer within that (ozk_matmul checks it)
@@ -440,27 +452,23 @@ int matmul_layout(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                                                 (void *)256, asl, nullptr, dummy3);
         ozk::SplitParams pb = make_split_params((const void *)256, o->bB, N, K, o->bt_strides,
                                                 L, o->alpha, (void *)256, bsl, nullptr, dummy3);
+        pa.Kp = pb.Kp = kp;
         const size_t wa = ozk::split_workspace_bytes(pa, ozk::plan_split(pa, dtype, sd), dtype, sd);
         const size_t wb = ozk::split_workspace_bytes(pb, ozk::plan_split(pb, dtype, sd), dtype, sd);
         scratch = wa > wb ? wa : wb;
     }
     o->scratch = off; off = align256(off + scratch);
     o->scratch_bytes = scratch;
-    // cross-GEMM view of the slices (a batch-1 split is broadcast); they are
-    // K-contiguous from a 256-byte aligned base, so only a row length that is
-    // not a multiple of 16 bytes needs the packed copy
-    const int64_t ga[4] = {o->bA == 1 ? 0 : L * M * K, M * K, K, 1};
-    const int64_t gb[4] = {o->bB == 1 ? 0 : L * N * K, N * K, 1, K};
+    // cross-GEMM view of the slices (a batch-1 split is broadcast)
+    const int64_t ga[4] = {o->bA == 1 ? 0 : L * M * kp, M * kp, kp, 1};
+    const int64_t gb[4] = {o->bB == 1 ? 0 : L * N * kp, N * kp, 1, kp};
     const int64_t gsa[3] = {o->bA == 1 ? 0 : L * M, M, 1};
     const int64_t gsb[3] = {o->bB == 1 ? 0 : L * N, N, 1};
     for (int t = 0; t < 4; ++t) { o->ga[t] = ga[t]; o->gb[t] = gb[t]; }
     for (int t = 0; t < 3; ++t) { o->gsa[t] = gsa[t]; o->gsb[t] = gsb[t]; }
-    const int64_t pk = pack_bytes((const void *)256, ga, batch, L, M, K, (int)ss, false) +
-                       pack_bytes((const void *)256, gb, batch, L, N, K, (int)ss, true);
-    o->pack = off; off = align256(off + (size_t)pk);
-    // the split-K buffers of a grid too small to fill the chip follow the
-    // pack region (the cross-GEMM runs without them when they are missing)
-    const int64_t kp = round_up(K * ss, 16) / ss;
+    // the split-K buffers of a grid too small to fill the chip (the cross-GEMM
+    // runs without them when they are missing)
+    o->sk = off;
     o->splitk = splitk_need(batch, M, N, K, L, sd, M * kp, kp, N * kp, kp, dtype);
     o->total = off + o->splitk;
     return OZK_OK;
@@ -520,15 +528,18 @@ int ozk_matmul_pairs(const void *A, const int64_t a_strides[3], const void *B,
     if (!workspace || workspace_bytes < lay.total - lay.splitk || (uintptr_t)workspace % 256 != 0)
         return OZK_ERR_WORKSPACE;
     char *ws = (char *)workspace;
-    const int64_t asl[4] = {L * M * K, M * K, K, 1}, bsl[4] = {L * N * K, N * K, K, 1};
+    const int64_t kp = lay.kp;
+    const int64_t asl[4] = {L * M * kp, M * kp, kp, 1}, bsl[4] = {L * N * kp, N * kp, kp, 1};
     const int64_t asc[3] = {L * M, M, 1}, bsc[3] = {L * N, N, 1};
     int e;
     // split B through its transposed view, then A (ozaki_triton.py:588-599)
     ozk::SplitParams pb = make_split_params(B, lay.bB, N, K, lay.bt_strides, L, lay.alpha,
                                             ws + lay.b_sl, bsl, (float *)(ws + lay.b_sc), bsc);
+    pb.Kp = kp;
     const ozk::SplitPlan plan_b = ozk::plan_split(pb, dtype, slice_dtype);
     ozk::SplitParams pa = make_split_params(A, lay.bA, M, K, a_strides, L, lay.alpha,
                                             ws + lay.a_sl, asl, (float *)(ws + lay.a_sc), asc);
+    pa.Kp = kp;
     const ozk::SplitPlan plan_a = ozk::plan_split(pa, dtype, slice_dtype);
     if (ozk::split_workspace_bytes(pb, plan_b, dtype, slice_dtype) > lay.scratch_bytes ||
         ozk::split_workspace_bytes(pa, plan_a, dtype, slice_dtype) > lay.scratch_bytes)
@@ -557,10 +568,10 @@ int ozk_matmul_pairs(const void *A, const int64_t a_strides[3], const void *B,
         if ((e = record(events, 1, st)) != OZK_OK) return e;
         if (hipError_t he = ozk::launch_split_pair(pa, plan_a, pb, plan_b, dtype, slice_dtype, st))
             return hip_status(he);
-    } else if (ozk::split_duo_ok(plan_a, plan_b, dtype)) {
-        // B's strips and A's row blocks in one launch (the same event rule)
+    } else if (ozk::split_fused_ok(pa, plan_a, pb, plan_b, dtype)) {
+        // both operands in one launch (the same event rule)
         if ((e = record(events, 1, st)) != OZK_OK) return e;
-        if (hipError_t he = ozk::launch_split_duo(pa, plan_a, pb, plan_b, dtype, slice_dtype, st))
+        if (hipError_t he = ozk::launch_split_fused(pa, plan_a, pb, plan_b, dtype, slice_dtype, st))
             return hip_status(he);
     } else {
         if (hipError_t he = ozk::launch_split(pb, plan_b, dtype, slice_dtype, st))
@@ -574,7 +585,7 @@ int ozk_matmul_pairs(const void *A, const int64_t a_strides[3], const void *B,
     e = cross_gemm_impl(ws + lay.a_sl, lay.ga, ws + lay.b_sl, lay.gb,
                         (const float *)(ws + lay.a_sc), lay.gsa, (const float *)(ws + lay.b_sc),
                         lay.gsb, batch, M, N, K, L, slice_dtype, pairs, C, dtype, c_strides,
-                        ws + lay.pack, workspace_bytes - lay.pack, stream, split_fail);
+                        ws + lay.sk, workspace_bytes - lay.sk, stream, split_fail, true);
     if (e != OZK_OK) return e;
     return record(events, 3, st);
 }

@@ -49,28 +49,16 @@ OZK_DEV double pow2d(int e) {
     return __longlong_as_double((long long)(e + 1023) << 52);
 }
 
-// Single round-to-nearest-even conversion of a binary64 value to binary16 (bit
-// pattern), written with integer arithmetic: one rounding from fp64, which a
-// conversion through fp32 would not give.
-OZK_DEV uint32_t f64_to_f16_bits(double x) {
-    uint64_t u = (uint64_t)__double_as_longlong(x);
-    uint32_t s = (uint32_t)((u >> 48) & 0x8000u);
-    int be = (int)((u >> 52) & 0x7FF);
-    uint64_t m = u & 0xFFFFFFFFFFFFFull;
-    if (be == 0x7FF) return s | (m ? 0x7E00u : 0x7C00u);
-    if (be == 0) return s;
-    uint64_t sig = (1ull << 52) | m;
-    int e = be - 1023;
-    int qe = (e < -14 ? -14 : e) - 10;
-    int shift = qe - (e - 52);
-    if (shift > 63) return s;
-    uint64_t n = sig >> shift;
-    uint64_t rem = sig & ((1ull << shift) - 1ull);
-    uint64_t half = 1ull << (shift - 1);
-    if (rem > half || (rem == half && (n & 1ull))) ++n;
-    uint32_t b = (e <= -14) ? (uint32_t)n : (uint32_t)(((e + 14) << 10) + (int)n);
-    if (b >= 0x7C00u) b = 0x7C00u;
-    return s | b;
+// Single round-to-nearest-even conversion of a binary64 value to binary16, as
+// two conversions: the low word of the mantissa becomes a sticky bit of the
+// high one, which leaves 21 significant bits, exact in binary32 (below 2^-126
+// the result is zero either way), and two more than a rounding to binary16's
+// 11 bits needs to be the rounding of the original value.
+OZK_DEV _Float16 f64_to_f16(double x) {
+    const uint64_t u = (uint64_t)__double_as_longlong(x);
+    const uint32_t sticky = (uint32_t)u != 0u ? 1u : 0u;
+    const uint32_t hi = (uint32_t)(u >> 32) | sticky;
+    return (_Float16)(float)__longlong_as_double((long long)((uint64_t)hi << 32));
 }
 // Single round-to-nearest-even conversion of a binary64 value to bfloat16 (bit
 // pattern).  bfloat16 has binary32's exponent range and 8 significant bits:
@@ -103,19 +91,5 @@ OZK_DEV uint32_t f32_to_bf16_bits(float x) {
     return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
 OZK_DEV float bf16_bits_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
-
-// exact binary16 -> binary32 (every binary16 value is a binary32 value)
-OZK_DEV float f16_bits_to_f32(uint32_t h) {
-    uint32_t s = (h & 0x8000u) << 16;
-    uint32_t be = (h >> 10) & 0x1Fu;
-    uint32_t m = h & 0x3FFu;
-    if (be == 0x1F) return __uint_as_float(s | 0x7F800000u | (m << 13));
-    if (be == 0) {
-        // subnormal: m * 2^-24, exact in binary32
-        float v = (float)m * 5.9604644775390625e-08f;
-        return s ? -v : v;
-    }
-    return __uint_as_float(s | ((be + 112u) << 23) | (m << 13));
-}
 
 }  // namespace ozk

@@ -44,6 +44,9 @@ struct SplitParams {
     int64_t ss_b, ss_l, ss_r, ss_k;
     float *scales;
     int64_t cs_b, cs_l, cs_r;
+    int64_t Kp;    // elements a slice row is written to, K or more: zeros beyond K
+    int cols;      // split_fused_kernel: the operand's columns, not its rows, are strided
+    int x_code;    // ... and the dtype code of X
     float *resid;  // workspace: exchange words of the cooperative kernels, the
                    // transposed operand [batch, rows, K] (transpose + row path) or
                    // the fp32 copy of a narrow input
@@ -57,10 +60,11 @@ struct SplitParams {
 
 enum SplitPath {
     kSplitRows = 0,
-    kSplitStrip = 1,
+    kSplitStrip = 1,   // columns, whole in one workgroup
     kSplitGeneric = 2,
     kSplitTransposeRows = 3,
-    kSplitConvert = 4,  // narrow input: exact fp32 copy in the workspace, then the fp32 plan
+    kSplitConvert = 4,  // narrow input, too long to convert as it is loaded: exact fp32
+                        // copy in the workspace, then the fp32 plan
     kSplitCoop = 5      // column strips of 128-byte row segments cut along K, the level
                         // maxima combined through the workspace
 };
@@ -95,11 +99,12 @@ bool split_pair_ok(const SplitPlan &plan_a, const SplitPlan &plan_b, int x_dtype
 hipError_t launch_split_pair(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
                              const SplitPlan &plan_b, int x_dtype, int slice_dtype,
                              hipStream_t stream);
-// both splits in one launch where B takes the 256-lane strip kernel and A a
-// 256-lane row configuration
-bool split_duo_ok(const SplitPlan &plan_a, const SplitPlan &plan_b, int x_dtype);
-hipError_t launch_split_duo(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
-                            const SplitPlan &plan_b, int x_dtype, int slice_dtype, hipStream_t st);
+// both splits in one launch where both take split_fused_kernel and neither its
+// wide column groups
+bool split_fused_ok(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
+                    const SplitPlan &plan_b, int x_dtype);
+hipError_t launch_split_fused(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
+                              const SplitPlan &plan_b, int x_dtype, int slice_dtype, hipStream_t st);
 
 // Sticky device status (per device): bit 0 is set when a cooperative split
 // wait gave up (the split's scales are then NaN).  read_device_status waits
