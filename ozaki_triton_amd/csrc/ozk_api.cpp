@@ -568,7 +568,7 @@ int ozk_matmul_pairs(const void *A, const int64_t a_strides[3], const void *B,
         if ((e = record(events, 1, st)) != OZK_OK) return e;
         if (hipError_t he = ozk::launch_split_pair(pa, plan_a, pb, plan_b, dtype, slice_dtype, st))
             return hip_status(he);
-    } else if (ozk::split_fused_ok(pa, plan_a, pb, plan_b, dtype)) {
+    } else if (ozk::split_fused_ok(plan_a, plan_b)) {
         // both operands in one launch (the same event rule)
         if ((e = record(events, 1, st)) != OZK_OK) return e;
         if (hipError_t he = ozk::launch_split_fused(pa, plan_a, pb, plan_b, dtype, slice_dtype, st))

@@ -99,10 +99,8 @@ bool split_pair_ok(const SplitPlan &plan_a, const SplitPlan &plan_b, int x_dtype
 hipError_t launch_split_pair(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
                              const SplitPlan &plan_b, int x_dtype, int slice_dtype,
                              hipStream_t stream);
-// both splits in one launch where both take split_fused_kernel and neither its
-// wide column groups
-bool split_fused_ok(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
-                    const SplitPlan &plan_b, int x_dtype);
+// both splits in one launch where both take split_fused_kernel
+bool split_fused_ok(const SplitPlan &plan_a, const SplitPlan &plan_b);
 hipError_t launch_split_fused(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
                               const SplitPlan &plan_b, int x_dtype, int slice_dtype, hipStream_t st);
 

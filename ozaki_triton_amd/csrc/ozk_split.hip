@@ -487,21 +487,20 @@ hipError_t launch_split_pair(const SplitParams &pa, const SplitPlan &plan_a,
     return with_slice(slice_dtype, [&](auto s) { return s.pair(pa, plan_a, pb, st); });
 }
 
-bool split_fused_ok(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
-                    const SplitPlan &plan_b, int x_dtype) {
-    if (debug_overrides().split != kForceSplitNone || !fused_plan(plan_a) || !fused_plan(plan_b) ||
-        plan_a.variant != plan_b.variant)
-        return false;
-    const SplitParams qa = fused_params(pa, plan_a, x_dtype), qb = fused_params(pb, plan_b, x_dtype);
-    return fused_width(qa, plan_a.variant, x_dtype) < 2 && fused_width(qb, plan_b.variant, x_dtype) < 2;
+bool split_fused_ok(const SplitPlan &plan_a, const SplitPlan &plan_b) {
+    return debug_overrides().split == kForceSplitNone && fused_plan(plan_a) && fused_plan(plan_b) &&
+           plan_a.variant == plan_b.variant;
 }
 
 hipError_t launch_split_fused(const SplitParams &pa, const SplitPlan &plan_a, const SplitParams &pb,
                               const SplitPlan &plan_b, int x_dtype, int slice_dtype,
                               hipStream_t st) {
+    if (!split_fused_ok(plan_a, plan_b)) return hipErrorInvalidValue;
     if (pa.batch * pa.rows == 0 || pb.batch * pb.rows == 0 || pa.L == 0) return hipSuccess;
     const SplitParams qa = fused_params(pa, plan_a, x_dtype), qb = fused_params(pb, plan_b, x_dtype);
-    const int width = qa.cols || qb.cols;
+    const int wa = fused_width(qa, plan_a.variant, x_dtype);
+    const int wb = fused_width(qb, plan_b.variant, x_dtype);
+    const int width = wa > wb ? wa : wb;
     return with_slice(slice_dtype, [&](auto s) {
         return s.fused(&qb, &qa, plan_a.variant, width, x_dtype, st);
     });

@@ -466,8 +466,15 @@ OZK_DEV void split_row(const SplitParams &p, int64_t xrow, int64_t srow, int K, 
             for (int u = 0; u < 4; ++u) asm volatile("" : "+v"(w[ch * 4 + u]));
         }
     };
-    level(0, std::true_type{}, v);
-    for (int l = 1; l < p.L; ++l) level(l, std::false_type{}, w);
+    if constexpr (std::is_same<V, float>::value) {
+        // one body for every level: less code to fetch
+#pragma unroll
+        for (int e = 0; e < NE; ++e) w[e] = v[e];
+        for (int l = 0; l < p.L; ++l) level(l, std::false_type{}, w);
+    } else {
+        level(0, std::true_type{}, v);
+        for (int l = 1; l < p.L; ++l) level(l, std::false_type{}, w);
+    }
 }
 
 // The body of the row kernel for row block `block`; red: LDS for the row maxima.
@@ -656,8 +663,18 @@ OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, 
                 for (int u = 0; u < VEC; ++u) asm volatile("" : "+v"(w[g][dk][u]));
         }
     };
-    level(0, std::true_type{}, v);
-    for (int l = 1; l < p.L; ++l) level(l, std::false_type{}, w);
+    if constexpr (std::is_same<V, float>::value) {
+#pragma unroll
+        for (int g = 0; g < NQ; ++g)
+#pragma unroll
+            for (int dk = 0; dk < 4; ++dk)
+#pragma unroll
+                for (int u = 0; u < VEC; ++u) w[g][dk][u] = v[g][dk][u];
+        for (int l = 0; l < p.L; ++l) level(l, std::false_type{}, w);
+    } else {
+        level(0, std::true_type{}, v);
+        for (int l = 1; l < p.L; ++l) level(l, std::false_type{}, w);
+    }
 }
 
 template <typename XC, typename ST, int NT, int SEG, int NQ>
@@ -708,25 +725,25 @@ __global__ __launch_bounds__(NT) void split_cols_kernel(SplitParams p) {
 struct FusedSplit {
     SplitParams op[2];
 };
-// (GW = 0: columns only; SEG = 0: rows only)
+// (SEG = 0: rows only)
 template <typename XC, typename ST, int NT, int GW, int NC, int SEG, int NQ>
 __global__ __launch_bounds__(NT) void split_fused_kernel(FusedSplit f, int64_t n0) {
     const int which = (int64_t)blockIdx.x >= n0;
     const SplitParams &p = f.op[which];
     const int64_t g = (int64_t)blockIdx.x - (which ? n0 : 0);
-    constexpr int RPB = GW > 0 ? NT / (64 * GW) : 1;
+    constexpr int RPB = NT / (64 * GW);
     __shared__ union {
         ColsShared<NT, (SEG > 0 ? SEG : 1), In<XC>::VEC> cols;
-        float rows[2][RPB][GW > 0 ? GW : 1];
+        float rows[2][RPB][GW];
     } sh;
     if constexpr (SEG > 0) {
-        if (GW == 0 || p.cols) {
+        if (p.cols) {
             split_cols_body<XC, ST, NT, SEG, NQ>(
                 p, xcd_remap(g, which ? (int64_t)gridDim.x - n0 : n0), sh.cols);
             return;
         }
     }
-    if constexpr (GW > 0) split_rows_body<XC, ST, GW, RPB, NC>(p, g, sh.rows);
+    split_rows_body<XC, ST, GW, RPB, NC>(p, g, sh.rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -1172,14 +1189,14 @@ static hipError_t launch_long(const SplitParams &p, const SplitPlan &plan, hipSt
 }
 
 // split_fused_kernel's configurations <NT, GW, NC, SEG, NQ> by class of K
-// (<= 256 << cls) and kind: rows only, narrow column groups (with rows or
-// columns of the other operand in the launch), or wide ones, in a launch of
-// their own: the registers they take would leave the rows' workgroups two
-// waves a SIMD (4096^2 f32 -> 2 f16, rows and wide columns: 80 us in one
-// launch, 64 in two).  A 16-byte piece of a row costs a whole 128-byte line
-// between L2 and the CU, so wider pieces win wherever their fewer, larger
-// groups still fill the chip.  Columns alone, us, N columns, f64 into 4 int8 / f32 into 2 fp16
-// slices (in brackets the 256- or 512-lane 16-byte strips of before this kernel):
+// (<= 256 << cls) and kind: rows only, narrow column groups or wide ones.  A
+// 16-byte piece of a row costs a whole 128-byte line between L2 and the CU, so
+// wider pieces win wherever their fewer, larger groups still fill the chip;
+// groups that hold more rows a lane would leave the rows' workgroups of the
+// same launch two waves a SIMD (<512,4,4,4,8> at K = 4096: 34 us against 39
+// where B is 16 times A, 60 against 50 where they are alike).  Columns alone,
+// us, N columns, f64 into 4 int8 / f32 into 2 fp16 slices (in brackets the
+// 256- or 512-lane 16-byte strips of before this kernel):
 //   K =  256 <256,4,1>  N = 1024  4.8 / 4.3   8192  9.4 / 5.9 [13.2 / 7.8]
 //   K =  512 <256,2,1>  N = 1024  5.9 / 4.3   8192 14.5 / 10.1 [20.2 / 12.9]
 //   K = 1024 <256,2,2>  N = 1024  6.7 / 5.3   8192 33.1 / 15.5 [39.5 / 19.1]
@@ -1189,12 +1206,16 @@ static hipError_t launch_long(const SplitParams &p, const SplitPlan &plan, hipSt
 //   K = 4096 <256,1,4>  N =  512 12.1 / 8.9 [14.6 / 10.0]
 //     wide   <512,2,4>  N = 2048 35.5 / 15.9   8192 118.8 / 79.5 [152.9 / 96.5]
 //   K = 8192 <512,1,4>  N = 2048 73.0 / 51.1 [97.5 / 58.4]
+// Rows and columns in one launch, narrow / wide: 4096^2 f64 -> 5 int8 115 / 108,
+// 4096^2 f32 -> 2 fp16 68 / 66, f64 -> 4 int8 2048 rows and 4096 columns of
+// 2048 41.9 / 39.9, 4096 and 4096 of 1024 27.9 / 24.5 (two launches: 120,
+// 67, 47, 28).
 enum { kNoCols = 0, kNarrowCols = 1, kWideCols = 2 };
 template <typename XC, typename ST, int NT, int GW, int NC, int SEG, int NQ>
 static hipError_t launch_fused_cfg(const FusedSplit &f, int n, hipStream_t st) {
     auto blocks = [](const SplitParams &p) -> int64_t {
         constexpr int SW = SEG > 0 ? SEG * In<XC>::VEC : 1;
-        constexpr int RPB = GW > 0 ? NT / (64 * GW) : 1;
+        constexpr int RPB = NT / (64 * GW);
         return p.cols ? p.batch * ((p.rows + SW - 1) / SW) : (p.batch * p.rows + RPB - 1) / RPB;
     };
     const int64_t n0 = blocks(f.op[0]);
@@ -1218,14 +1239,14 @@ static hipError_t launch_fused_x(const FusedSplit &f, int n, int cls, int width,
     case 10: OZK_FUSED(256, 4, 2, 2, 4);
     case 12: OZK_FUSED(256, 4, 4, 0, 0);
     case 13: OZK_FUSED(256, 4, 4, 1, 4);
-    case 14: OZK_FUSED(512, 0, 0, 2, 4);
+    case 14: OZK_FUSED(512, 4, 4, 2, 4);
     case 15: OZK_FUSED(256, 4, 8, 0, 0);
     case 16: OZK_FUSED(512, 4, 8, 1, 4);
     }
     if constexpr (F64) {
         switch (3 * cls + width) {
-        case 8: OZK_FUSED(256, 0, 0, 4, 4);
-        case 11: OZK_FUSED(512, 0, 0, 4, 4);
+        case 8: OZK_FUSED(256, 1, 4, 4, 4);
+        case 11: OZK_FUSED(512, 4, 2, 4, 4);
         }
     }
 #undef OZK_FUSED

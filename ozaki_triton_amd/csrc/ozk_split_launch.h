@@ -67,8 +67,7 @@ hipError_t launch_poison(const SplitParams &p, const uint64_t *status, hipStream
 
 template <typename ST> struct SplitLaunch {
     // p0 and (unless null) p1 by split_fused_kernel, K of class cls, columns
-    // by the groups of this width (0: no columns, 1: narrow, 2: wide, columns
-    // only)
+    // by the groups of this width (0: no columns, 1: narrow, 2: wide)
     static hipError_t fused(const SplitParams *p0, const SplitParams *p1, int cls, int width,
                             int x_dtype, hipStream_t st);
     // one fp64 / fp32 operand by any other kernel
