@@ -149,10 +149,34 @@ OZK_DEV void resolve_split_fail(GemmParams &p) {
         __hip_atomic_fetch_or(p.dev_status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-OZK_DEV int64_t xcd_remap_gemm(int64_t g, int64_t n) {
-    const int64_t q = n / 8;
+OZK_DEV uint32_t xcd_remap_gemm(uint32_t g, uint32_t n) {
+    const uint32_t q = n / 8;
     if (g >= q * 8) return g;
     return (g % 8) * q + g / 8;
+}
+
+// Tile g of a grid (batch, then groups of group_m tile rows, column by column
+// within a group; group_m a power of two).  The tile count is the grid's, so
+// everything fits 32 bits: a 64-bit division is a chain of some hundred
+// dependent instructions, and three of them held back every workgroup's first
+// load by about a microsecond.
+struct TileAt {
+    int64_t bidx, m0, n0;
+};
+template <int BM, int BN> OZK_DEV TileAt tile_at(const GemmParams &p, uint32_t g, int group_m) {
+    const uint32_t tiles_m = (uint32_t)((p.M + BM - 1) / BM);
+    const uint32_t tiles_n = (uint32_t)((p.N + BN - 1) / BN);
+    uint32_t b = 0, t = g;
+    if (p.batch > 1) {
+        b = g / (tiles_m * tiles_n);
+        t = g - b * (tiles_m * tiles_n);
+    }
+    const uint32_t first_m = (t / tiles_n) & ~((uint32_t)group_m - 1);
+    const uint32_t in_group = t - first_m * tiles_n;
+    const uint32_t left = tiles_m - first_m;
+    const uint32_t gsz = left < (uint32_t)group_m ? left : (uint32_t)group_m;
+    const uint32_t tn = in_group / gsz, tm = first_m + in_group - tn * gsz;
+    return {(int64_t)b, (int64_t)tm * BM, (int64_t)tn * BN};
 }
 
 template <int N, typename F> OZK_DEV void static_for(F &&f) {
@@ -232,19 +256,8 @@ __global__ __launch_bounds__(256, 1) void cross_gemm_kernel(GemmParams p, int gr
     const int wm = wave >> 1, wn = wave & 1;
     const int h = lane >> 5, lr = lane & 31;
 
-    // ---- tile coordinates ----
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
-    const int64_t g = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const int64_t kbytes = p.K * ES;
     const int nkb = (int)((kbytes + kRowBytes - 1) / kRowBytes);
@@ -503,18 +516,8 @@ __global__ __launch_bounds__(256, 1) void cross_gemm_dma_kernel(GemmParams p, in
     const int wm = wave >> 1, wn = wave & 1;
     const int h = lane >> 5, lr = lane & 31;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
-    const int64_t g = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -815,18 +818,8 @@ __global__ __launch_bounds__(256 * G, 1) void cross_gemm_kstep_kernel(GemmParams
     const int ks = wave & 3, grp = wave >> 2;   // K step of every stage, pair group
     const int h = lane >> 5, lr = lane & 31;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
-    const int64_t g = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -1138,18 +1131,8 @@ __global__ __launch_bounds__(512, 1) void cross_gemm_pair_kernel(GemmParams p, i
     const int wm = blk >> 1, wn = blk & 1;
     const int h = lane >> 5, lr = lane & 31;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
-    const int64_t g = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -1422,22 +1405,14 @@ __global__ __launch_bounds__(512, 1) void cross_gemm_ring_kernel(GemmParams p, i
     const int wm = blk >> 1, wn = blk & 1;
     const int h = lane >> 5, lr = lane & 31;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
     // split-K: workgroup g0 is K range g0 % S of tile g0 / S
     const int S = p.ksplit > 1 ? p.ksplit : 1;
-    const int64_t g0 = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int krange = (int)(g0 % S);
-    const int64_t g = g0 / S;
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const uint32_t g0 = xcd_remap_gemm(blockIdx.x, gridDim.x);
+    const uint32_t gt = S > 1 ? g0 / (uint32_t)S : g0;
+    const int krange = (int)(g0 - gt * (uint32_t)S);
+    const int64_t g = gt;
+    const TileAt at = tile_at<BM, BN>(p, gt, group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb_all = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -1800,22 +1775,14 @@ __global__ __launch_bounds__(512, 1) void cross_gemm_wide_kernel(GemmParams p, i
     const int wm = wave >> 2, wn = wave & 3;
     const int h = lane >> 5, lr = lane & 31;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
     // split-K: workgroup g0 is K range g0 % S of tile g0 / S
     const int S = p.ksplit > 1 ? p.ksplit : 1;
-    const int64_t g0 = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int krange = (int)(g0 % S);
-    const int64_t g = g0 / S;
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const uint32_t g0 = xcd_remap_gemm(blockIdx.x, gridDim.x);
+    const uint32_t gt = S > 1 ? g0 / (uint32_t)S : g0;
+    const int krange = (int)(g0 - gt * (uint32_t)S);
+    const int64_t g = gt;
+    const TileAt at = tile_at<BM, BN>(p, gt, group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb_all = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -2115,18 +2082,8 @@ __global__ __launch_bounds__(512, 1) void cross_gemm_wide4_kernel(GemmParams p, 
     const int a_rstep = last_i ? 32 : BM;
     const int h = lane >> 5, lr = lane & 31;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
-    const int64_t g = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -2517,18 +2474,8 @@ __global__ __launch_bounds__(512, 1) void cross_gemm_wide4q_kernel(GemmParams p,
     const int wy = last_i ? wave - 6 : (wave & 1);
     const int wx = last_i ? 0 : (wave >> 1);
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
-    const int64_t g = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -2925,22 +2872,14 @@ __global__ __launch_bounds__(512, 1) void cross_gemm_wideq_kernel(GemmParams p, 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 2, wn = wave & 3;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
     // split-K: workgroup g0 is K range g0 % S of tile g0 / S
     const int S = p.ksplit > 1 ? p.ksplit : 1;
-    const int64_t g0 = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int krange = (int)(g0 % S);
-    const int64_t g = g0 / S;
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const uint32_t g0 = xcd_remap_gemm(blockIdx.x, gridDim.x);
+    const uint32_t gt = S > 1 ? g0 / (uint32_t)S : g0;
+    const int krange = (int)(g0 - gt * (uint32_t)S);
+    const int64_t g = gt;
+    const TileAt at = tile_at<BM, BN>(p, gt, group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb_all = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -3334,22 +3273,14 @@ __global__ __launch_bounds__(512, 1) void cross_gemm_ringq_kernel(GemmParams p, 
     const int blk = wave & 3, grp = wave >> 2;   // block; pair group
     const int wm = blk >> 1, wn = blk & 1;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
     // split-K: workgroup g0 is K range g0 % S of tile g0 / S
     const int S = p.ksplit > 1 ? p.ksplit : 1;
-    const int64_t g0 = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int krange = (int)(g0 % S);
-    const int64_t g = g0 / S;
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const uint32_t g0 = xcd_remap_gemm(blockIdx.x, gridDim.x);
+    const uint32_t gt = S > 1 ? g0 / (uint32_t)S : g0;
+    const int krange = (int)(g0 - gt * (uint32_t)S);
+    const int64_t g = gt;
+    const TileAt at = tile_at<BM, BN>(p, gt, group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb_all = (int)((kbytes + kDmaRB - 1) / kDmaRB);
@@ -3801,18 +3732,8 @@ __global__ __launch_bounds__(256, 1) void cross_gemm_soloq_kernel(GemmParams p, 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wx = wave >> 1, wy = wave & 1;
 
-    const int64_t tiles_m = (p.M + BM - 1) / BM;
-    const int64_t tiles_n = (p.N + BN - 1) / BN;
-    const int64_t tiles = tiles_m * tiles_n;
-    const int64_t g = xcd_remap_gemm(blockIdx.x, (int64_t)gridDim.x);
-    const int64_t bidx = g / tiles;
-    const int64_t t = g % tiles;
-    const int64_t width = (int64_t)group_m * tiles_n;
-    const int64_t first_m = (t / width) * group_m;
-    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
-    const int64_t tm = first_m + (t % width) % gsz;
-    const int64_t tn = (t % width) / gsz;
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb = (int)((kbytes + kDmaRB - 1) / kDmaRB);
