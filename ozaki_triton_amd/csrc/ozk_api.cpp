@@ -112,7 +112,8 @@ int64_t pack_bytes(const void *ptr, const int64_t s[4], int64_t batch, int L, in
                     (zero_padded || (K * es) % 16 == 0);
     if (ok || rows == 0 || K == 0 || L == 0) return 0;
     const int64_t kp = round_up(K * es, 16) / es;
-    return round_up(batch * L * rows * kp * es, 256);
+    // (a broadcast operand is packed once)
+    return round_up((s[0] == 0 ? 1 : batch) * L * rows * kp * es, 256);
 }
 
 }  // namespace
@@ -292,13 +293,15 @@ static int cross_gemm_impl(const void *A_slices, const int64_t a_strides[4], con
     const int64_t kp = round_up(K * es, 16) / es;
     char *ws = (char *)workspace;
 
+    const ozk::PackParams pka{A_slices, a_strides[0], a_strides[1], a_strides[2], a_strides[3],
+                              ws, a_strides[0] == 0 ? 1 : batch, num_splits, M, K, kp, es};
+    const ozk::PackParams pkb{B_slices, b_strides[0], b_strides[1], b_strides[3], b_strides[2],
+                              ws + abytes, b_strides[0] == 0 ? 1 : batch, num_splits, N, K, kp, es};
+    if (ozk::launch_pack(abytes > 0 ? &pka : nullptr, bbytes > 0 ? &pkb : nullptr, st) != hipSuccess)
+        return OZK_ERR_LAUNCH;
     if (abytes > 0) {
-        ozk::PackParams pk{A_slices, a_strides[0], a_strides[1], a_strides[2], a_strides[3],
-                           ws, batch, num_splits, M, K, kp, es};
-        hipError_t e = ozk::launch_pack(pk, st);
-        if (e != hipSuccess) return OZK_ERR_LAUNCH;
         p.A = ws;
-        p.as_b = num_splits * M * kp;
+        p.as_b = a_strides[0] == 0 ? 0 : num_splits * M * kp;
         p.as_l = M * kp;
         p.as_m = kp;
         ws += abytes;
@@ -309,12 +312,8 @@ static int cross_gemm_impl(const void *A_slices, const int64_t a_strides[4], con
         p.as_m = a_strides[2];
     }
     if (bbytes > 0) {
-        ozk::PackParams pk{B_slices, b_strides[0], b_strides[1], b_strides[3], b_strides[2],
-                           ws, batch, num_splits, N, K, kp, es};
-        hipError_t e = ozk::launch_pack(pk, st);
-        if (e != hipSuccess) return OZK_ERR_LAUNCH;
         p.B = ws;
-        p.bs_b = num_splits * N * kp;
+        p.bs_b = b_strides[0] == 0 ? 0 : num_splits * N * kp;
         p.bs_l = N * kp;
         p.bs_n = kp;
     } else {

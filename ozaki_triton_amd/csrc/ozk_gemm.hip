@@ -6,27 +6,111 @@
 namespace ozk {
 
 // ---------------------------------------------------------------------------
-// Pack kernel: any-stride slices -> K-contiguous, 16-byte padded rows.
+// Pack kernel: any-stride slices -> K-contiguous, 16-byte padded rows, one or
+// both operands in a launch, a broadcast operand once.  Bound by the bytes it
+// moves and the launch; one element a lane with three 64-bit divisions each
+// ran at a tenth of that (both operands, us: 64 and 128 rows of 7228 in 4 int8
+// slices 23.0 -> 7.0; 3 x 1051 and 5473 rows of 239 in 4 fp16 slices 63.8 ->
+// 11.5).  Three ways, by the source's strides:
+//   K-contiguous rows: a lane makes one 16-byte piece of a row from one load
+//   (element alignment is enough), the row's last piece element by element;
+//   row-contiguous (the [K, N] layout): 64 x 64 tiles turned in the LDS;
+//   any other: one element a lane.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void pack_kernel(PackParams p) {
-    const int64_t total = p.batch * p.L * p.rows * p.Kp;
-    for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total;
-         idx += (int64_t)gridDim.x * 256) {
-        const int64_t k = idx % p.Kp;
-        int64_t rest = idx / p.Kp;
-        const int64_t r = rest % p.rows;
-        rest /= p.rows;
-        const int64_t l = rest % p.L;
-        const int64_t b = rest / p.L;
-        const int64_t so = b * p.s_b + l * p.s_l + r * p.s_r + k * p.s_k;
-        if (p.esize == 1) {
-            ((int8_t *)p.dst)[idx] = (k < p.K) ? ((const int8_t *)p.src)[so] : (int8_t)0;
-        } else if (p.esize == 2) {
-            ((uint16_t *)p.dst)[idx] = (k < p.K) ? ((const uint16_t *)p.src)[so] : (uint16_t)0;
-        } else {
-            ((uint32_t *)p.dst)[idx] = (k < p.K) ? ((const uint32_t *)p.src)[so] : 0u;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4a1 __attribute__((ext_vector_type(4), aligned(1)));
+constexpr int kPackTile = 64;
+
+enum { kPackRows = 0, kPackTiles = 1, kPackAny = 2 };
+// the first two count rows in 32 bits
+__host__ __device__ inline int pack_way(const PackParams &p) {
+    if (p.batch * p.L * p.rows >= (int64_t)1 << 31) return kPackAny;
+    return p.s_k == 1 ? kPackRows : p.s_r == 1 ? kPackTiles : kPackAny;
+}
+
+// the source offset of row `row` of the operand (batch, slice, row)
+template <typename I> OZK_DEV int64_t pack_row(const PackParams &p, I row) {
+    const I rows = (I)p.rows, L = (I)p.L;
+    const I bl = row / rows, r = row - bl * rows;
+    const I b = bl / L, l = bl - b * L;
+    return (int64_t)b * p.s_b + (int64_t)l * p.s_l + (int64_t)r * p.s_r;
+}
+
+template <typename E>
+OZK_DEV void pack_body(const PackParams &p, uint32_t block, uint32_t nblocks, E (*tile)[kPackTile + 1]) {
+    constexpr int PE = 16 / (int)sizeof(E);   // elements of a 16-byte piece
+    const uint64_t nrow = (uint64_t)(p.batch * p.L * p.rows);
+    const int way = pack_way(p);
+    if (way == kPackRows) {
+        const uint32_t pieces = (uint32_t)(p.Kp / PE);
+        const uint64_t total = nrow * pieces;
+        for (uint64_t i = (uint64_t)block * 256 + threadIdx.x; i < total; i += (uint64_t)nblocks * 256) {
+            const uint32_t row = total >> 32 ? (uint32_t)(i / pieces) : (uint32_t)i / pieces;
+            const int64_t k = (int64_t)(i - (uint64_t)row * pieces) * PE;
+            const E *src = (const E *)p.src + pack_row(p, row) + k;
+            u32x4 v;
+            if (k + PE <= p.K) {
+                v = *(const u32x4a1 *)src;
+            } else {
+                E e[PE];
+#pragma unroll
+                for (int u = 0; u < PE; ++u) e[u] = k + u < p.K ? src[u] : (E)0;
+                __builtin_memcpy(&v, e, 16);
+            }
+            ((u32x4 *)p.dst)[i] = v;
+        }
+    } else if (way == kPackTiles) {
+        const uint32_t tk = (uint32_t)((p.Kp + kPackTile - 1) / kPackTile);
+        const uint32_t tr = (uint32_t)((p.rows + kPackTile - 1) / kPackTile);
+        const uint64_t total = (uint64_t)p.batch * p.L * tk * tr;
+        const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+        for (uint64_t t = block; t < total; t += nblocks) {
+            const uint32_t bl = (uint32_t)(t / ((uint64_t)tk * tr));
+            const uint32_t in = (uint32_t)(t - (uint64_t)bl * tk * tr);
+            const int64_t k0 = (int64_t)(in / tr) * kPackTile, r0 = (int64_t)(in % tr) * kPackTile;
+            const int64_t so = (int64_t)(bl / (uint32_t)p.L) * p.s_b + (int64_t)(bl % (uint32_t)p.L) * p.s_l;
+#pragma unroll 4
+            for (int k = y; k < kPackTile; k += 4)
+                tile[k][x] = k0 + k < p.K && r0 + x < p.rows
+                                 ? ((const E *)p.src)[so + (k0 + k) * p.s_k + r0 + x]
+                                 : (E)0;
+            __syncthreads();
+            for (int q = threadIdx.x; q < kPackTile * (kPackTile / PE); q += 256) {
+                const int r = q / (kPackTile / PE), k = (q % (kPackTile / PE)) * PE;
+                if (r0 + r < p.rows && k0 + k < p.Kp) {
+                    E e[PE];
+#pragma unroll
+                    for (int u = 0; u < PE; ++u) e[u] = tile[k + u][r];
+                    u32x4 v;
+                    __builtin_memcpy(&v, e, 16);
+                    *(u32x4 *)((E *)p.dst + ((int64_t)bl * p.rows + r0 + r) * p.Kp + k0 + k) = v;
+                }
+            }
+            __syncthreads();
+        }
+    } else {
+        const uint64_t total = nrow * (uint64_t)p.Kp;
+        for (uint64_t i = (uint64_t)block * 256 + threadIdx.x; i < total; i += (uint64_t)nblocks * 256) {
+            const uint64_t row = i / (uint64_t)p.Kp;
+            const int64_t k = (int64_t)(i - row * (uint64_t)p.Kp);
+            ((E *)p.dst)[i] = k < p.K ? ((const E *)p.src)[pack_row(p, row) + k * p.s_k] : (E)0;
         }
     }
+}
+
+struct PackPair {
+    PackParams op[2];
+};
+// the first n0 workgroups pack op[0], the others op[1]
+__global__ __launch_bounds__(256) void pack_kernel(PackPair f, unsigned n0) {
+    __shared__ uint32_t tile[kPackTile * (kPackTile + 1)];
+    const int which = blockIdx.x >= n0;
+    const PackParams &p = f.op[which];
+    const uint32_t block = blockIdx.x - (which ? n0 : 0);
+    const uint32_t nblocks = which ? gridDim.x - n0 : n0;
+    if (p.esize == 1) pack_body<uint8_t>(p, block, nblocks, (uint8_t(*)[kPackTile + 1])tile);
+    else if (p.esize == 2) pack_body<uint16_t>(p, block, nblocks, (uint16_t(*)[kPackTile + 1])tile);
+    else pack_body<uint32_t>(p, block, nblocks, (uint32_t(*)[kPackTile + 1])tile);
 }
 
 // num_splits == 0: the reference's kernel stores its zero-initialised outer
@@ -53,12 +137,24 @@ hipError_t launch_zero_c(const GemmParams &p, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_pack(const PackParams &p, hipStream_t st) {
-    const int64_t total = p.batch * p.L * p.rows * p.Kp;
-    if (total == 0) return hipSuccess;
-    int64_t blocks = (total + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL(pack_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p);
+hipError_t launch_pack(const PackParams *pa, const PackParams *pb, hipStream_t st) {
+    // workgroups of an operand: one 16-byte piece a lane, one tile, or four
+    // elements a lane
+    auto blocks = [](const PackParams &p) -> int64_t {
+        const int64_t pieces = p.batch * p.L * p.rows * (p.Kp * p.esize / 16);
+        const int way = pack_way(p);
+        const int64_t n = way == kPackRows ? (pieces + 255) / 256
+                          : way == kPackTiles
+                              ? p.batch * p.L * ((p.rows + 63) / 64) * ((p.Kp + 63) / 64)
+                              : (p.batch * p.L * p.rows * p.Kp + 1023) / 1024;
+        return n < 65536 ? n : 65536;
+    };
+    const PackParams *first = pa ? pa : pb;
+    if (!first) return hipSuccess;
+    const PackPair f{{*first, pa && pb ? *pb : *first}};
+    const int64_t n0 = blocks(f.op[0]), n1 = pa && pb ? blocks(f.op[1]) : 0;
+    if (n0 + n1 == 0) return hipSuccess;
+    hipLaunchKernelGGL(pack_kernel, dim3((unsigned)(n0 + n1)), dim3(256), 0, st, f, (unsigned)n0);
     return hipGetLastError();
 }
 

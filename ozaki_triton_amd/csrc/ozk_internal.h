@@ -200,6 +200,7 @@ struct PackParams {
     int64_t batch, L, rows, K, Kp;
     int esize;
 };
-hipError_t launch_pack(const PackParams &p, hipStream_t stream);
+// (either may be null; both go in one launch)
+hipError_t launch_pack(const PackParams *pa, const PackParams *pb, hipStream_t stream);
 
 }  // namespace ozk
