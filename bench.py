@@ -239,9 +239,9 @@ def planned_gemm_kernel(batch, M, N, K, L, sdt, pairs="all"):
 def gemm_kernel_symbol(plan, L, sdt):
     """Name of the kernel function a planned cross-GEMM launches: the
     launchers take the 16 x 16 MFMA forms ("...q") of the ring (two slices),
-    wide, wide4 and solo configurations for the slice dtypes benchmarked
+    wide, wide4, solo and short configurations for the slice dtypes benchmarked
     here (int8, fp16)."""
-    q = plan in ("ring", "wide", "wide4", "solo")
+    q = plan in ("ring", "wide", "wide4", "solo", "short")
     return f"cross_gemm_{plan}{'q' if q else ''}_kernel"
 
 
@@ -557,7 +557,7 @@ def main():
     for _ in range(warmup - done - 1):
         _ozaki_matmul_impl(A, B, L, slice_dtype, False, None, max_splits=8, pairs=args.pairs)
     # the last warmup step with all four events: are the splits one launch
-    # (split_pair_kernel / split_duo_kernel)?  Then the B phase's two events
+    # (split_pair_kernel / split_fused_kernel)?  Then the B phase's two events
     # fall at one point
     _ozaki_matmul_impl(A, B, L, slice_dtype, False, events[0], max_splits=8, pairs=args.pairs)
     torch.cuda.synchronize()

@@ -167,10 +167,10 @@ def device_status(clear: bool = True, stream=None) -> int:
 
 class forced_kernels:
     """Context manager for tests: force the cross-GEMM kernel (`gemm`: "staged",
-    "dma", "pair", "ring", "wide", "wide4", "solo"), its split-K ranges
-    (`ksplit`, ring and wide kernels; 1: none) and / or the split kernel
-    (`split`: "coop", "strip", "transpose", "generic", "rows", "rowscoop") of
-    the calls this host thread makes inside it, and optionally make every
+    "dma", "pair", "ring", "wide", "wide4", "solo", "kstep", "kstep2",
+    "short"), its split-K ranges (`ksplit`, ring and wide kernels; 1: none) and
+    / or the split kernel (`split`: "coop", "strip", "transpose", "generic",
+    "rows", "rowscoop") of the calls this host thread makes inside it, and optionally make every
     cooperative split wait give up at once (`coop_timeout`).  Restores the
     defaults on exit."""
 

@@ -297,6 +297,41 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
     // (1, 128, 2048, 4096) and 256^2 x 4096, int8 and fp16, 2-4 slices:
     // 3-9% faster)
     if (plan.kind == kGemmKStep && L >= 2) plan.kind = kGemmKStep2;
+    // The short-K kernel (two workgroups of small tiles per CU).  Its tiles
+    // move more bytes per MFMA than the other kernels', so up to a length of a
+    // row of K, in bytes, and on grids that occupy the CUs.  Cross-GEMM alone
+    // (kernel trace), the other kernel's time over this one's, int8 into fp64
+    // by bytes of K, in brackets fp16 into fp32 at as many bytes:
+    //   1 slice, from 512 tiles, any K: 4096^2 128 bytes 2.1 (2.7), 4096 1.6
+    //     (1.7); 2048^2, 256 tiles, 1024 1.00 (0.94), 2048 0.95 (0.86)
+    //   2 slices, from 256 tiles, to 1024 bytes: 4096^2 64 1.44 (1.50), 1024
+    //     1.10 (1.17), 4096 0.93; 1536^2, 288 tiles, 1.48 to 1.15 (1.37 to
+    //     1.15); 1024 x 1536, 192 tiles, 1.08 to 0.95 (0.94 to 0.84)
+    //   2, triangle, from 256 tiles, to 4096 bytes: 4096^2 128 2.8 (2.6), 2048
+    //     1.7 (1.55), 4096 1.5; 1536^2 1.54 to 1.20 (1.41 to 1.19); 1024 x 1536
+    //     1.11 to 0.95 (0.93 to 0.75)
+    //   3, triangle, to 512: 4096^2 64 1.35 (1.35), 512 1.17 (1.21), 2048
+    //     (1.00); 2048^2 512 1.02 (1.02), 1024 0.94 (0.93); 1024^2 1.11 to 1.04
+    //     (1.10 to 1.08).  All pairs stay: 4096^2 64 1.09 (1.03), 512 1.01
+    //     (0.95); 2048^2 0.99 (0.91 to 1.04)
+    //   4, to 512: 4096^2 64 1.32 (1.31), 512 1.08 (1.12), 1024 1.01 (0.95);
+    //     1024^2 1.10 to 1.05 (1.17 to 1.08); 8192^2 x 256 513 -> 433 us
+    //   4, triangle, to 512, or 1024 in two rounds and more: 4096^2 64 1.60
+    //     (1.66), 1024 1.16 (1.21), 2048 1.01 (1.04); 1024^2, 512 tiles, 512
+    //     1.08 (1.15), 1024 0.97 (0.99)
+    //   5, triangle, to 512: 4096^2 64 1.43 (1.49), 512 1.13 (1.19), 1024 0.94
+    //     (1.05); 1024^2 1.19 to 1.13 (1.29 to 1.11)
+    const int64_t kbytes = p.K * es;
+    const int64_t short_bm = L <= 2 ? 128 : 64, short_bn = L == 1 ? 128 : L <= 3 ? 64 : 32;
+    const int64_t short_tiles =
+        p.batch * ((p.M + short_bm - 1) / short_bm) * ((p.N + short_bn - 1) / short_bn);
+    const bool short_has = fits && slice_dtype != 1 && (p.tri ? L <= 5 : L <= 4 && L != 3);
+    const bool short_kernel =
+        short_has && !kstep &&
+        (L == 1   ? short_tiles >= 2 * kCUs
+         : L == 2 ? short_tiles >= kCUs && kbytes <= (p.tri ? 4096 : 1024)
+                  : kbytes <= (L == 4 && p.tri && short_tiles > 2 * kCUs ? 1024 : 512));
+    if (short_kernel) plan.kind = kGemmShort;
     const int force = debug_overrides().gemm;
     auto forced = [&](int kind) { return force == kind; };
     if (p.tri && L >= 2) {
@@ -305,7 +340,8 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
         // grids), wide4 at L = 4 where its rounds rule holds, the LDS-DMA
         // kernel at L = 2, the one-wave-per-SIMD kernel otherwise at L = 4
         // (below) and at L = 5 (int8 / fp16 / bf16; fp32 slices: the LDS-DMA
-        // kernel at L = 4, the pair-split kernel over all i-rows at L = 5).
+        // kernel at L = 4, the pair-split kernel over all i-rows at L = 5);
+        // a short K on the short-K kernel (above).
         // Measured, cross-GEMM alone, full-range random int8 slices, pair /
         // solo at L = 5: 8192^3 8.12 / 6.99 ms,
         // 4096^2 x 8192 2.04 / 1.75, 2048^2 x 8192 0.487 / 0.399, 1024^2 x
@@ -325,6 +361,7 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
         const bool solo4 = L == 4 && slice_dtype != 1 && !(nt(1, 1) <= kCUs && nkb_all >= 256);
         plan.kind = !fits     ? kGemmStaged
                     : kstep   ? kGemmKStep2
+                    : short_kernel ? kGemmShort
                     : L == 3  ? kGemmWide
                     : wide4   ? kGemmWide4
                     : solo4   ? kGemmSolo
@@ -341,8 +378,11 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
                 plan.kind = kGemmKStep;
             else if (fits && forced(kGemmKStep2) && L >= 2) plan.kind = kGemmKStep2;
             else if (fits && forced(kGemmSolo) && L == 4 && slice_dtype != 1) plan.kind = kGemmSolo;
+            else if (forced(kGemmShort) && short_has) plan.kind = kGemmShort;
         } else if (fits && forced(kGemmSolo) && solo5) {
             plan.kind = kGemmSolo;
+        } else if (forced(kGemmShort) && short_has) {
+            plan.kind = kGemmShort;
         } else if (fits && forced(kGemmPair)) {
             plan.kind = kGemmPair;
         }
@@ -374,6 +414,7 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
     else if (fits && forced(kGemmKStep)) plan.kind = (L == 4 && slice_dtype == 1) ? plan.kind : kGemmKStep;
     else if (fits && forced(kGemmKStep2) && L >= 2) plan.kind = kGemmKStep2;
     else if (fits && forced(kGemmSolo) && L == 4 && slice_dtype != 1) plan.kind = kGemmSolo;
+    else if (forced(kGemmShort) && short_has) plan.kind = kGemmShort;
     // 96 x 64 tiles: groups of 4 tile rows (C3: 7.12-7.16 ms against 7.21-7.23
     // with 8, 7.33-7.35 with 16; cross-GEMM alone, one box)
     if (plan.kind == kGemmWide4) plan.group_m = 4;

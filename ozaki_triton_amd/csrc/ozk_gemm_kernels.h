@@ -132,6 +132,20 @@ OZK_DEV void store_c(const GemmParams &p, int64_t idx, float v) {
     }
 }
 
+// A lane's stores to C from row row0 and column col0 on: one 64-bit address,
+// stepped by uniform products.
+struct StoreC {
+    int64_t base;
+    int mleft, nleft;
+    OZK_DEV StoreC(const GemmParams &p, int64_t b, int64_t row0, int64_t col0)
+        : base(b * p.cs_b + row0 * p.cs_m + col0 * p.cs_n),
+          mleft((int)(p.M - row0 < 1024 ? p.M - row0 : 1024)),
+          nleft((int)(p.N - col0 < 1024 ? p.N - col0 : 1024)) {}
+    template <typename OA> OZK_DEV void put(const GemmParams &p, int dr, int dc, OA v) const {
+        if (dr < mleft && dc < nleft) store_c(p, base + (dr * p.cs_m + dc * p.cs_n), v);
+    }
+};
+
 // Kernel entry: reads the status words of the cooperative splits that ran
 // before on the same stream (complete when the kernel starts) into p.failed,
 // and records a failure in the device's sticky status (one lane).
@@ -4033,6 +4047,216 @@ __global__ __launch_bounds__(256, 1) void cross_gemm_soloq_kernel(GemmParams p, 
 }
 
 // ---------------------------------------------------------------------------
+// The short-K kernel: two workgroups of 4 waves per CU, for contractions of a
+// few stages.  There a tile of the kernels above spends more on its set-up,
+// its first stage and its epilogue than on the K loop, one after the other
+// (a 96 x 64 tile of wide4q at K = 256, fp64 C, cycles: set-up 1,000, first
+// stages 3,400, K loop 8,600, epilogue 13,100), and its one workgroup per CU
+// leaves the matrix cores idle meanwhile.  Here a second workgroup runs its K
+// loop under the first one's epilogue and loads.  Tiles, by num_splits: 128 x
+// 128 (1), 128 x 64 (2), 64 x 64 (3, triangle), 64 x 32 (4, and 5 on the
+// triangle), a 2 x 2 grid of waves, each wave every pair of its block: at most 144 accumulator
+// registers of the 256 a wave has at two waves per SIMD, and one stage of 128
+// bytes of K (32 to 60 KB).  The
+// stage is not double-buffered: the other workgroup fills the wait.  Fragments,
+// swizzle and MFMAs as in cross_gemm_wideq_kernel, the epilogue tile by tile
+// (16 x 16), in the reference's order.  Smaller tiles move more bytes per MFMA,
+// so longer contractions keep the kernels above (plan_gemm).
+// ---------------------------------------------------------------------------
+template <int L_> struct ShortShape {
+    static constexpr int L = L_;
+    static constexpr int RM = L <= 2 ? 4 : 2;                     // 16-row tiles of a wave
+    static constexpr int RN = L == 1 ? 4 : L <= 3 ? 2 : 1;        // 16-column tiles
+    static constexpr int BM = 32 * RM, BN = 32 * RN;
+    static constexpr int A_BYTES = L * BM * kDmaRB, B_BYTES = L * BN * kDmaRB;
+    static constexpr int WA = A_BYTES / 1024, WB = B_BYTES / 1024;   // 1 KB windows
+    static constexpr int LA = WA / 4, LB = WB / 4;                   // ... of a wave
+    static constexpr int NSC = L * (BM + BN);                        // scales
+    static constexpr int LDS_BYTES = A_BYTES + B_BYTES + NSC * 4;
+    static_assert(WA % 4 == 0 && WB % 4 == 0 && (BM / 8) % 2 == 0 && (BN / 8) % 4 == 0,
+                  "whole windows per wave, of the wave's parity");
+    static_assert(2 * LDS_BYTES <= 160 * 1024, "two workgroups per CU");
+};
+
+template <typename ST, int L, typename AccT, bool TRI>
+__global__ __launch_bounds__(256, 2) void cross_gemm_shortq_kernel(GemmParams p, int group_m,
+                                                                   uint32_t a_records,
+                                                                   uint32_t b_records) {
+    resolve_split_fail(p);
+    using Sh = ShortShape<L>;
+    using MF = Mfma16<ST>;
+    using Acc = typename MF::Acc;
+    using OA = AccT;
+    using PS = Pairs<L, TRI>;
+    constexpr int BM = Sh::BM, BN = Sh::BN, RM = Sh::RM, RN = Sh::RN;
+    constexpr int ES = (int)sizeof(ST);
+    constexpr uint32_t kOOB = 0x80000000u;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    float *const sa_lds = (float *)(smem + Sh::A_BYTES + Sh::B_BYTES), *const sb_lds = sa_lds + L * BM;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
+    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
+
+    const uint32_t kbytes = (uint32_t)(p.K * ES);
+    const int nkb = (int)((kbytes + kDmaRB - 1) / kDmaRB);
+    const int nkb_full = (int)(kbytes / kDmaRB);
+
+    const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)((const char *)p.A + bidx * p.as_b * ES), (short)0, (int)a_records, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rB = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)((const char *)p.B + bidx * p.bs_b * ES), (short)0, (int)b_records, 0x00020000);
+
+    // the tile's scales: loaded first, written to the LDS under the first
+    // stage's DMA
+    constexpr int SQ = (Sh::NSC + 255) / 256;
+    float sc[SQ];
+#pragma unroll
+    for (int q = 0; q < SQ; ++q) {
+        const int e = q * 256 + tid;
+        const bool isa = e < L * BM;
+        const int f = isa ? e : e - L * BM;
+        const int s = isa ? f / BM : f / BN;
+        const int64_t rc = isa ? m0 + f % BM : n0 + f % BN;
+        const bool ok = e < Sh::NSC && rc < (isa ? p.M : p.N);
+        const float *src = isa ? p.sa + bidx * p.sas_b + s * p.sas_l + rc * p.sas_m
+                               : p.sb + bidx * p.sbs_b + s * p.sbs_l + rc * p.sbs_n;
+        sc[q] = ok ? *src : 0.0f;
+    }
+
+    // Stage DMA: windows of 8 rows as in wideq; wave w takes the A windows w +
+    // 4 q (q < LA) and B windows w + 4 q (q < LB), all of its parity.
+    const int c0 = (lane & 7) ^ (lane >> 4) ^ ((wave & 1) ? 4 : 0);   // logical chunk of this lane
+    const uint32_t lane_a = (uint32_t)((lane >> 3) * p.as_m * ES) + (uint32_t)c0 * 16;
+    const uint32_t lane_b = (uint32_t)((lane >> 3) * p.bs_n * ES) + (uint32_t)c0 * 16;
+    auto stage_dma = [&](int kb) {
+        const int kleft = (int)kbytes - kb * kDmaRB;
+        auto window = [&](bool isa, int w) {
+            const int per = (isa ? BM : BN) / 8;   // windows of a slice
+            const int s = w / per;
+            const int64_t first = (isa ? m0 : n0) + 8 * (w % per);
+            const uint32_t ub = (uint32_t)__builtin_amdgcn_readfirstlane(
+                (int)((uint32_t)(((int64_t)s * (isa ? p.as_l : p.bs_l) +
+                                  first * (isa ? p.as_m : p.bs_n)) * ES) + (uint32_t)kb * kDmaRB));
+            const int64_t left = (isa ? p.M : p.N) - first;
+            auto *ldsp = (__attribute__((address_space(3))) void *)(smem + (isa ? 0 : Sh::A_BYTES) + w * 1024);
+            const uint32_t lsrc = isa ? lane_a : lane_b;
+            if (left >= 8 && kb < nkb_full) {
+                if (isa) __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, ldsp, 16, lsrc, (int)ub, 0, 0);
+                else __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, ldsp, 16, lsrc, (int)ub, 0, 0);
+            } else {
+                const uint32_t vo = ((lane >> 3) < left && c0 * 16 < kleft) ? lsrc + ub : kOOB;
+                if (isa) __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, ldsp, 16, vo, 0, 0, 0);
+                else __builtin_amdgcn_raw_ptr_buffer_load_lds(rB, ldsp, 16, vo, 0, 0, 0);
+            }
+        };
+#pragma unroll
+        for (int q = 0; q < Sh::LA; ++q) window(true, wave + 4 * q);
+#pragma unroll
+        for (int q = 0; q < Sh::LB; ++q) window(false, wave + 4 * q);
+    };
+    if (nkb > 0) stage_dma(0);
+#pragma unroll
+    for (int q = 0; q < SQ; ++q)
+        if (q * 256 + tid < Sh::NSC) sa_lds[q * 256 + tid] = sc[q];
+
+    const int qrow = lane & 15, key = (qrow >> 1) & 7;
+    using lds_cptr = const __attribute__((address_space(3))) char *;
+    const lds_cptr lds0 = (lds_cptr)smem;
+    const int a_org = wm * 16 * RM * kDmaRB, b_org = Sh::A_BYTES + wn * 16 * RN * kDmaRB;
+
+    Acc acc[PS::N][RM][RN];
+#pragma unroll
+    for (int n = 0; n < PS::N; ++n)
+#pragma unroll
+        for (int r = 0; r < RM; ++r)
+#pragma unroll
+            for (int c = 0; c < RN; ++c) acc[n][r][c] = MF::zero();
+
+    for (int kb = 0; kb < nkb; ++kb) {
+        // the stage has landed: this wave's DMA, then every wave's
+        wait_vmcnt<0>();
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        exec_barrier();
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const int lane_rd = qrow * kDmaRB + (((4 * kk + (lane >> 4)) ^ key) << 4);
+            const lds_cptr ra = lds0 + a_org + lane_rd, rb = lds0 + b_org + lane_rd;
+            i32x4 fa[L][RM];
+#pragma unroll
+            for (int i = 0; i < L; ++i)
+#pragma unroll
+                for (int r = 0; r < RM; ++r)
+                    fa[i][r] = *(const __attribute__((address_space(3))) i32x4 *)(
+                        ra + (i * BM + 16 * r) * kDmaRB);
+            static_for<L>([&](auto j_) {
+                constexpr int j = decltype(j_)::value;
+#pragma unroll
+                for (int c = 0; c < RN; ++c) {
+                    const i32x4 fb = *(const __attribute__((address_space(3))) i32x4 *)(
+                        rb + (j * BN + 16 * c) * kDmaRB);
+                    static_for<L>([&](auto i_) {
+                        constexpr int i = decltype(i_)::value;
+                        if constexpr (PS::kept(i, j)) {
+                            constexpr int n = PS::first(i) + j;
+#pragma unroll
+                            for (int r = 0; r < RM; ++r)
+                                acc[n][r][c] = MF::mfma(fa[i][r], fb, acc[n][r][c]);
+                        }
+                    });
+                }
+            });
+        }
+        if (kb + 1 < nkb) {
+            // every wave has read the stage: its buffer is free
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            exec_barrier();
+            stage_dma(kb + 1);
+        }
+    }
+    if (nkb == 0) {   // the scales' writes
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        exec_barrier();
+    }
+
+    // ---- epilogue: ordered outer accumulation, ozaki_triton.py:420-452 ----
+    const int eq = lane & 15, eg = lane >> 4;
+    const StoreC st(p, bidx, m0 + wm * 16 * RM + 4 * eg, n0 + wn * 16 * RN + eq);
+#pragma unroll
+    for (int c = 0; c < RN; ++c) {
+        float sbv[L];
+#pragma unroll
+        for (int j = 0; j < L; ++j) sbv[j] = sb_lds[j * BN + (wn * RN + c) * 16 + eq];
+#pragma unroll
+        for (int r = 0; r < RM; ++r) {
+            OA out[4] = {(OA)0, (OA)0, (OA)0, (OA)0};
+            static_for<L>([&](auto i_) {
+                constexpr int i = decltype(i_)::value;
+                const f32x4 s4 = *(const f32x4 *)(sa_lds + i * BM + (wm * RM + r) * 16 + 4 * eg);
+                static_for<L>([&](auto j_) {
+                    constexpr int j = decltype(j_)::value;
+                    if constexpr (PS::kept(i, j)) {
+                        constexpr int n = PS::first(i) + j;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            // fl32(fl32(fl32(acc) * sa_i) * sb_j), summed i-major, j-minor
+                            const float t1 = MF::to_f32(acc[n][r][c][e]) * s4[e];
+                            out[e] = out[e] + (OA)(t1 * sbv[j]);
+                        }
+                    }
+                });
+            });
+#pragma unroll
+            for (int e = 0; e < 4; ++e) st.put(p, 16 * r + e, 16 * c, out[e]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Launch templates (host side)
 // ---------------------------------------------------------------------------
 // byte extent [0, bytes) one batch of a slice operand spans, or -1 if it does
@@ -4201,6 +4425,22 @@ static hipError_t launch_solo(const GemmParams &p, const GemmPlan &plan, hipStre
     }
 }
 
+template <typename ST, int L, typename AccT, bool TRI>
+static hipError_t launch_short(const GemmParams &p, const GemmPlan &plan, hipStream_t st) {
+    using Sh = ShortShape<L>;
+    auto kern = cross_gemm_shortq_kernel<ST, L, AccT, TRI>;
+    static std::atomic<uint64_t> lds_set{0};   // devices whose LDS limit is raised
+    if (hipError_t e = set_lds_limit((const void *)kern, Sh::LDS_BYTES, lds_set)) return e;
+    const int es = (int)sizeof(ST);
+    const int64_t ea = dma_extent(p.as_l, p.as_m, L, p.M, p.K, es);
+    const int64_t eb = dma_extent(p.bs_l, p.bs_n, L, p.N, p.K, es);
+    const int64_t tiles = p.batch * ((p.M + Sh::BM - 1) / Sh::BM) * ((p.N + Sh::BN - 1) / Sh::BN);
+    if (tiles == 0) return hipSuccess;
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(256), Sh::LDS_BYTES, st, p,
+                       plan.group_m, (uint32_t)ea, (uint32_t)eb);
+    return hipGetLastError();
+}
+
 // num_splits = 5..8: launches over consecutive i-rows (at most 16 pairs each,
 // so a wave group still holds 8 pairs), in i-major order, each continuing the
 // fp64 sum from C.  int8 / fp16 / bf16 slices with an fp64 outer accumulator.
@@ -4266,6 +4506,9 @@ static hipError_t launch_L(const GemmParams &p, const GemmPlan &plan, hipStream_
     }
     if constexpr (L >= 2 && L <= 4) {
         if (plan.kind == kGemmKStep2) return launch_kstep<ST, L, AccT, TRI, 2>(p, plan, st);
+    }
+    if constexpr ((TRI ? L <= 5 : L <= 4 && L != 3) && !std::is_same_v<ST, float>) {
+        if (plan.kind == kGemmShort) return launch_short<ST, L, AccT, TRI>(p, plan, st);
     }
     const int key = plan.mi * 10 + plan.ni;
     if constexpr (L == 1) {
