@@ -392,6 +392,20 @@ OZK_DEV void lds_barrier() {
     asm volatile("s_barrier" ::: "memory");
 }
 
+// a / b and its remainder (a >= 0, b > 0, uniform over the workgroup): in 32 bits
+// where they fit.  Every workgroup's first load waits for its row's batch and
+// row.
+struct Quot {
+    int64_t q, r;
+};
+OZK_DEV Quot quot(int64_t a, int64_t b) {
+    if (((uint64_t)(a | b) >> 32) == 0) {
+        const uint32_t q = (uint32_t)a / (uint32_t)b;
+        return {(int64_t)q, (int64_t)((uint32_t)a - q * (uint32_t)b)};
+    }
+    return {a / b, a % b};
+}
+
 // ---------------------------------------------------------------------------
 // Row-resident split.  Block = RPB groups of G = 64*GW lanes; group g owns
 // global row block*RPB + g.  Lane t of a group holds elements
@@ -488,8 +502,8 @@ OZK_DEV void split_rows_body(const SplitParams &p, int64_t block, float (*red)[R
     const int64_t nrows = p.batch * p.rows;
     const int64_t grow = block * RPB + grp;
     const bool off = grow >= nrows;
-    const int64_t b = off ? 0 : grow / p.rows;
-    const int64_t r = off ? 0 : grow % p.rows;
+    const Quot at = quot(off ? 0 : grow, p.rows);
+    const int64_t b = at.q, r = at.r;
     float *srow_scale = p.scales + b * p.cs_b + r * p.cs_r;
     auto smax = [&](float m, int l) { return row_max<GW, RPB>(m, red, l & 1, grp, t); };
     auto put = [&](int l, const LevelScale &c) {
@@ -687,8 +701,8 @@ OZK_DEV void split_cols_body(const SplitParams &p, int64_t sidx,
     const int tid = threadIdx.x;
     const int seg = tid % SEG, ro = tid / SEG;
     const int64_t nstr = (p.rows + SW - 1) / SW;
-    const int64_t b = sidx / nstr;
-    const int64_t col0 = (sidx % nstr) * SW, col = col0 + seg * VEC;
+    const Quot at = quot(sidx, nstr);
+    const int64_t b = at.q, col0 = at.r * SW, col = col0 + seg * VEC;
     const int ncol = (int)(p.rows - col < VEC ? p.rows - col : VEC);
     const bool col_ok = col0 + SW <= p.rows;
     const int64_t xb = b * p.xs_b + col + 4 * ro * p.xs_k;
@@ -811,8 +825,8 @@ OZK_DEV void split_coop_body(const SplitParams &p, uint64_t *slot, int P, uint32
     const int member = (int)(g % P);
     const int64_t grp = g / P;
     const int64_t nstr = (p.rows + SW - 1) / SW;
-    const int64_t b = grp / nstr;
-    const int64_t col0 = (grp % nstr) * SW;
+    const Quot at = quot(grp, nstr);
+    const int64_t b = at.q, col0 = at.r * SW;
     const int64_t mycol = col0 + seg * VEC;
     const int64_t kbase = (int64_t)member * (RPP * RPL) + 4 * ro;   // this lane's first row
     // of this lane's columns, those that exist; and its rows' limits
@@ -978,7 +992,8 @@ __global__ __launch_bounds__(64 * GW) void split_rows_coop_kernel(SplitParams p,
     const int64_t g = blockIdx.x;
     const int member = (int)(g % P);
     const int64_t grow = g / P;
-    const int64_t b = grow / p.rows, r = grow % p.rows;
+    const Quot at = quot(grow, p.rows);
+    const int64_t b = at.q, r = at.r;
     const int64_t kbase = (int64_t)member * CHR;
     const int kleft = (int)(p.K - kbase);    // this chunk's elements inside the row
     const int sleft = (int)(p.Kp - kbase);   // and inside the slice row
