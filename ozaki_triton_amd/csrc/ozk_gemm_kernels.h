@@ -530,8 +530,21 @@ __global__ __launch_bounds__(256, 1) void cross_gemm_dma_kernel(GemmParams p, in
     const int wm = wave >> 1, wn = wave & 1;
     const int h = lane >> 5, lr = lane & 31;
 
-    const TileAt at = tile_at<BM, BN>(p, xcd_remap_gemm(blockIdx.x, gridDim.x), group_m);
-    const int64_t bidx = at.bidx, m0 = at.m0, n0 = at.n0;
+    // (64-bit coordinates here, not tile_at: with those in 32 bits, 2048^2 x 512
+    // of 2 fp16 slices took 40.4 us against 35.9, of 1 slice 19.0 against 17.5;
+    // only grids of one round, 1536^2, gained, 3%)
+    const int64_t tiles_m = (p.M + BM - 1) / BM;
+    const int64_t tiles_n = (p.N + BN - 1) / BN;
+    const int64_t tiles = tiles_m * tiles_n;
+    const int64_t g = xcd_remap_gemm(blockIdx.x, gridDim.x);
+    const int64_t bidx = g / tiles;
+    const int64_t t = g % tiles;
+    const int64_t width = (int64_t)group_m * tiles_n;
+    const int64_t first_m = (t / width) * group_m;
+    const int64_t gsz = (tiles_m - first_m < group_m) ? (tiles_m - first_m) : group_m;
+    const int64_t tm = first_m + (t % width) % gsz;
+    const int64_t tn = (t % width) / gsz;
+    const int64_t m0 = tm * BM, n0 = tn * BN;
 
     const uint32_t kbytes = (uint32_t)(p.K * ES);
     const int nkb = (int)((kbytes + kDmaRB - 1) / kDmaRB);
