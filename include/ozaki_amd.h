@@ -124,6 +124,9 @@ int ozk_compute_split_bits(int64_t n, int slice_dtype, int dot_accum_dtype, int 
  * rows), plus a status word; an fp32 copy of a narrow input, or a transposed
  * copy of a long column operand.  The query sees no pointers: it sizes for
  * 16-byte aligned X and slices, and a call with other pointers needs no more.
+ * Operands that are not whole 16-byte pieces (K, pitch or alignment) run with
+ * less as well, slower: the exchange words and the transposed copy are then
+ * left out, an fp32 copy is not.
  */
 int ozk_split_workspace_bytes(int x_dtype, int64_t batch, int64_t rows, int64_t K,
                               const int64_t x_strides[3], int num_splits, int slice_dtype,
@@ -233,9 +236,10 @@ int ozk_matmul_pairs(const void *A, const int64_t a_strides[3], const void *B,
  * tight serving loops, harnesses that forbid hipMalloc): ozk_matmul with its
  * workspace taken from a library-owned device array of OZK_STATIC_SCRATCH_BYTES,
  * one per device, held until the process ends.  The caller still passes the
- * inputs and C.  A call that needs more than that, not counting the optional
- * split-K buffers (ozk_matmul_workspace_bytes() includes them), returns
- * OZK_ERR_TOO_LARGE before anything is enqueued; split-K buffers that do not
+ * inputs and C.  A call that needs more than that returns OZK_ERR_TOO_LARGE
+ * before anything is enqueued.  Not counted, though part of
+ * ozk_matmul_workspace_bytes(): the split-K buffers, and the scratch of
+ * operands that can do without (ozk_split); split-K buffers that do not
  * fit as well are left out (the same bits, from unsplit tiles).  The call allocates
  * nothing (no hipMalloc, hipFree or allocating library routine).  All calls on
  * one device share its array: calls that overlap on one device (other streams

@@ -94,6 +94,15 @@ int ozk_debug_split_kernel(const void *X, int x_dtype, int64_t batch, int64_t ro
                            const void *slices, const int64_t slice_strides[4],
                            const char **name_out, size_t *bytes_out);
 
+/*
+ * The workspace bytes, split-K buffers not counted, that ozk_matmul needs when
+ * the caller has `have` bytes: with too few for the plans of both operands,
+ * operands that can do without scratch (ozk_split) are planned without.
+ */
+int ozk_debug_matmul_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
+                               const int64_t a_strides[3], const int64_t b_strides[3],
+                               int num_splits, int slice_dtype, size_t have, size_t *bytes_out);
+
 #ifdef __cplusplus
 }
 #endif

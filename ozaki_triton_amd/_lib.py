@@ -55,6 +55,7 @@ EXPORTED_DEBUG = (
     "ozk_debug_gemm_kernel",
     "ozk_debug_gemm_kernel_pairs",
     "ozk_debug_split_kernel",
+    "ozk_debug_matmul_workspace",
 )
 
 _lib = None
@@ -136,6 +137,9 @@ def load() -> ctypes.CDLL:
     L.ozk_debug_split_kernel.argtypes = [vp, i32, i64, i64, i64, p64, i32, i32, vp, p64,
                                          ctypes.POINTER(ctypes.c_char_p), ctypes.POINTER(sz)]
     L.ozk_debug_split_kernel.restype = i32
+    L.ozk_debug_matmul_workspace.argtypes = [i32, i64, i64, i64, i64, p64, p64, i32, i32,
+                                             ctypes.c_size_t, ctypes.POINTER(ctypes.c_size_t)]
+    L.ozk_debug_matmul_workspace.restype = i32
     _lib = L
     return L
 

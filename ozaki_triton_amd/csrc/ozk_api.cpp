@@ -204,10 +204,12 @@ int ozk_split(const void *X, int x_dtype, int64_t batch, int64_t rows, int64_t K
     if (!X || !slices || !scales) return OZK_ERR_NULL;
     ozk::SplitParams p = make_split_params(X, batch, rows, K, x_strides, num_splits, alpha,
                                            slices, slice_strides, scales, scale_strides);
-    const ozk::SplitPlan plan = ozk::plan_split(p, x_dtype, slice_dtype);
+    const bool usable = workspace && (uintptr_t)workspace % 16 == 0;
+    const ozk::SplitPlan plan =
+        ozk::plan_split(p, x_dtype, slice_dtype, usable ? workspace_bytes : 0);
     const size_t need = ozk::split_workspace_bytes(p, plan, x_dtype, slice_dtype);
     if (need > 0) {
-        if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16 != 0)
+        if (!usable || workspace_bytes < need)
             return OZK_ERR_WORKSPACE;
         p.resid = (float *)workspace;
     }
@@ -399,9 +401,11 @@ struct MatmulLayout {
     int64_t ga[4], gb[4], gsa[3], gsb[3];           // cross-GEMM strides of the slices
 };
 
+// limit: the bytes the caller has (the queries: any); with fewer than the plans
+// of both operands need, those that can do without scratch are planned so
 int matmul_layout(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
                   const int64_t as[3], const int64_t bs[3], int L, int sd, int pairs,
-                  MatmulLayout *o) {
+                  MatmulLayout *o, size_t limit = SIZE_MAX) {
     if (!is_input_dtype(dtype) || !is_slice_dtype(sd)) return OZK_ERR_DTYPE;
     if (batch < 0 || M < 0 || N < 0 || K < 0) return OZK_ERR_SHAPE;
     // alpha for every num_splits, 0 included: the reference calls
@@ -452,9 +456,15 @@ int matmul_layout(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
         ozk::SplitParams pb = make_split_params((const void *)256, o->bB, N, K, o->bt_strides,
                                                 L, o->alpha, (void *)256, bsl, nullptr, dummy3);
         pa.Kp = pb.Kp = kp;
-        const size_t wa = ozk::split_workspace_bytes(pa, ozk::plan_split(pa, dtype, sd), dtype, sd);
-        const size_t wb = ozk::split_workspace_bytes(pb, ozk::plan_split(pb, dtype, sd), dtype, sd);
-        scratch = wa > wb ? wa : wb;
+        auto need = [&](size_t have) {
+            auto of = [&](const ozk::SplitParams &p) {
+                return ozk::split_workspace_bytes(p, ozk::plan_split(p, dtype, sd, have), dtype, sd);
+            };
+            const size_t wa = of(pa), wb = of(pb);
+            return wa > wb ? wa : wb;
+        };
+        scratch = need(SIZE_MAX);
+        if (align256(off + scratch) > limit) scratch = need(limit > off ? limit - off : 0);
     }
     o->scratch = off; off = align256(off + scratch);
     o->scratch_bytes = scratch;
@@ -509,7 +519,7 @@ int ozk_matmul_pairs(const void *A, const int64_t a_strides[3], const void *B,
     if (!a_strides || !b_strides || !c_strides) return OZK_ERR_NULL;
     MatmulLayout lay;
     const int lst = matmul_layout(dtype, batch, M, N, K, a_strides, b_strides, num_splits,
-                                  slice_dtype, pairs, &lay);
+                                  slice_dtype, pairs, &lay, workspace ? workspace_bytes : 0);
     if (lst != OZK_OK) return lst;
     if (batch * M * N == 0) return OZK_OK;
     if (!C) return OZK_ERR_NULL;
@@ -535,11 +545,11 @@ int ozk_matmul_pairs(const void *A, const int64_t a_strides[3], const void *B,
     ozk::SplitParams pb = make_split_params(B, lay.bB, N, K, lay.bt_strides, L, lay.alpha,
                                             ws + lay.b_sl, bsl, (float *)(ws + lay.b_sc), bsc);
     pb.Kp = kp;
-    const ozk::SplitPlan plan_b = ozk::plan_split(pb, dtype, slice_dtype);
+    const ozk::SplitPlan plan_b = ozk::plan_split(pb, dtype, slice_dtype, lay.scratch_bytes);
     ozk::SplitParams pa = make_split_params(A, lay.bA, M, K, a_strides, L, lay.alpha,
                                             ws + lay.a_sl, asl, (float *)(ws + lay.a_sc), asc);
     pa.Kp = kp;
-    const ozk::SplitPlan plan_a = ozk::plan_split(pa, dtype, slice_dtype);
+    const ozk::SplitPlan plan_a = ozk::plan_split(pa, dtype, slice_dtype, lay.scratch_bytes);
     if (ozk::split_workspace_bytes(pb, plan_b, dtype, slice_dtype) > lay.scratch_bytes ||
         ozk::split_workspace_bytes(pa, plan_a, dtype, slice_dtype) > lay.scratch_bytes)
         return OZK_ERR_WORKSPACE;
@@ -631,7 +641,7 @@ extern "C" int ozk_matmul_static(const void *A, const int64_t a_strides[3], cons
     if (!a_strides || !b_strides || !c_strides) return OZK_ERR_NULL;
     MatmulLayout lay;
     const int lst = matmul_layout(dtype, batch, M, N, K, a_strides, b_strides, num_splits,
-                                  slice_dtype, OZK_PAIRS_ALL, &lay);
+                                  slice_dtype, OZK_PAIRS_ALL, &lay, OZK_STATIC_SCRATCH_BYTES);
     if (lst != OZK_OK) return lst;
     if (batch * M * N == 0 || num_splits == 0)   // no workspace used
         return ozk_matmul(A, a_strides, B, b_strides, dtype, batch, M, N, K, num_splits,
@@ -710,6 +720,17 @@ int ozk_debug_coop_residency(int force, int *resident_out) {
     if (force >= 0) ozk::debug_overrides().coop_resident = force;
     if (resident_out) *resident_out = ozk::coop_resident_per_xcd();
     return OZK_OK;
+}
+
+int ozk_debug_matmul_workspace(int dtype, int64_t batch, int64_t M, int64_t N, int64_t K,
+                               const int64_t a_strides[3], const int64_t b_strides[3],
+                               int num_splits, int slice_dtype, size_t have, size_t *bytes_out) {
+    if (!bytes_out || !a_strides || !b_strides) return OZK_ERR_NULL;
+    MatmulLayout lay;
+    const int st = matmul_layout(dtype, batch, M, N, K, a_strides, b_strides, num_splits,
+                                 slice_dtype, OZK_PAIRS_ALL, &lay, have);
+    if (st == OZK_OK) *bytes_out = lay.total - lay.splitk;
+    return st;
 }
 
 int ozk_debug_gemm_kernel(int64_t batch, int64_t M, int64_t N, int64_t K, int num_splits,

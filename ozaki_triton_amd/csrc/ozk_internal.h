@@ -69,6 +69,9 @@ enum SplitPath {
                         // maxima combined through the workspace
 };
 
+// variant of kSplitConvert: the copy goes to the generic kernel
+constexpr int kConvertGeneric = 1;
+
 // Chooses the split kernel for p (x_dtype: 0 = f64, 1 = f32, 2 = f16,
 // 3 = bf16, 4 = i8; slice: 1 = f32, 2 = f16, 3 = bf16, 4 = i8).  Returns the path and, for the resident paths, the variant index.
 struct SplitPlan {
@@ -78,8 +81,10 @@ struct SplitPlan {
 // The plan depends on the pointers X and slices only through alignment.  The
 // workspace queries see no pointers and size for 256-byte aligned ones; a plan
 // for other pointers never needs more scratch than that (it falls back to the
-// generic kernel, which needs none).
-SplitPlan plan_split(const SplitParams &p, int x_dtype, int slice_dtype);
+// generic kernel, which needs none).  scratch: the bytes there are; an operand
+// that is not whole 16-byte pieces takes a plan without scratch where its own
+// needs more, any other keeps its plan (the caller refuses the call).
+SplitPlan plan_split(const SplitParams &p, int x_dtype, int slice_dtype, size_t scratch = SIZE_MAX);
 // scratch the plan needs: the exchange words of the cooperative kernels and
 // their status word, the transposed operand (transpose + row path), the fp32
 // copy of a narrow input (none for the row, strip and generic kernels)

@@ -308,8 +308,30 @@ static SplitPlan plan_split_raw(const SplitParams &p, int x_dtype, int slice_dty
 }
 
 
-SplitPlan plan_split(const SplitParams &p, int x_dtype, int slice_dtype) {
+// Operands that are not whole 16-byte pieces (K, row pitch, alignment) can do
+// without scratch: long ones take a cooperative or transposing plan where there
+// is scratch for it, else the generic kernel.  Callers that own a buffer of one
+// size (ozk_matmul_static, or ozk_split without a workspace) need no room for
+// them.  Whole operands must have what their plan needs.
+static bool scratch_optional(const SplitParams &p, int x_dtype, int slice_dtype) {
+    const int xsz = dtype_size(x_dtype), ssz = dtype_size(slice_dtype);
+    const bool slices_whole = p.ss_k == 1 && aligned(p.slices, 4 * ssz) && p.ss_r % 4 == 0 &&
+                              p.ss_l % 4 == 0 && p.ss_b % 4 == 0;
+    if (p.K % 4 != 0 || !slices_whole) return true;
+    if (x_dtype >= 2) return false;   // split from a whole fp32 copy
+    return !aligned(p.X, 16) ||
+           (p.xs_k == 1 && ((p.xs_r * xsz) % 16 != 0 || (p.xs_b * xsz) % 16 != 0));
+}
+// the plan without scratch of its own (a narrow input keeps its fp32 copy)
+static SplitPlan plan_without_scratch(int x_dtype) {
+    return x_dtype >= 2 ? SplitPlan{kSplitConvert, kConvertGeneric} : SplitPlan{kSplitGeneric, 0};
+}
+
+SplitPlan plan_split(const SplitParams &p, int x_dtype, int slice_dtype, size_t scratch) {
     const SplitPlan plan = plan_split_raw(p, x_dtype, slice_dtype);
+    const size_t need = split_workspace_bytes(p, plan, x_dtype, slice_dtype);
+    if (need > scratch && scratch_optional(p, x_dtype, slice_dtype))
+        return plan_without_scratch(x_dtype);
     if (aligned(p.X, 16) && aligned(p.slices, 16)) return plan;   // the aligned plan
     // other pointers: no more scratch than the workspace queries reserve for
     // aligned ones, which see no pointers (the generic kernel needs none)
@@ -317,15 +339,15 @@ SplitPlan plan_split(const SplitParams &p, int x_dtype, int slice_dtype) {
     q.X = (const void *)(uintptr_t)256;
     q.slices = (void *)(uintptr_t)256;
     const SplitPlan ref = plan_split_raw(q, x_dtype, slice_dtype);
-    if (split_workspace_bytes(p, plan, x_dtype, slice_dtype) >
-        split_workspace_bytes(q, ref, x_dtype, slice_dtype))
-        return {kSplitGeneric, 0};
+    if (need > split_workspace_bytes(q, ref, x_dtype, slice_dtype))
+        return plan_without_scratch(x_dtype);
     return plan;
 }
 
 // plan of the fp32 copy of a narrow input (its X is the 16-byte aligned
 // workspace: `aligned` in plan_split must see an aligned pointer)
-static SplitPlan converted_plan(const SplitParams &p, int slice_dtype) {
+static SplitPlan converted_plan(const SplitParams &p, const SplitPlan &plan, int slice_dtype) {
+    if (plan.variant == kConvertGeneric) return {kSplitGeneric, 0};
     SplitParams q = converted_params(p);
     q.X = (const void *)(uintptr_t)256;
     return plan_split(q, 1, slice_dtype);
@@ -335,7 +357,7 @@ size_t split_workspace_bytes(const SplitParams &p, const SplitPlan &plan, int x_
                              int slice_dtype) {
     const int64_t n = p.batch * p.rows * p.K;
     if (plan.path == kSplitConvert) {
-        const SplitPlan inner = converted_plan(p, slice_dtype);
+        const SplitPlan inner = converted_plan(p, plan, slice_dtype);
         const size_t in = split_workspace_bytes(converted_params(p), inner, 1, slice_dtype);
         return in ? round256((size_t)(n * 4)) + in : (size_t)(n * 4);
     }
@@ -455,7 +477,7 @@ hipError_t launch_split(const SplitParams &p, const SplitPlan &plan, int x_dtype
         SplitParams q = converted_params(p);
         q.X = T;
         q.resid = (float *)((char *)T + round256((size_t)(p.batch * p.rows * p.K) * 4));
-        return launch_split(q, plan_split(q, 1, slice_dtype), 1, slice_dtype, st);
+        return launch_split(q, converted_plan(p, plan, slice_dtype), 1, slice_dtype, st);
     }
     if (plan.path == kSplitTransposeRows) {
         // workspace: [batch, rows, K], then the shared row kernel's exchange words
