@@ -289,6 +289,14 @@ OZK_DEV void load_some(const void *x, int64_t i, int left, int code, typename In
     }
 }
 
+// ... all of them, or none (zeros)
+template <typename XC, int N>
+OZK_DEV void load_quad(const void *x, int64_t i, bool there, int code, typename In<XC>::V *v) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) v[u] = (typename In<XC>::V)0;
+    if (there) Load<XC>::template vec<N>(x, i, code, v);
+}
+
 // Store 4 consecutive slice values (k .. k+3) of one row.
 typedef uint32_t u32a1 __attribute__((aligned(1)));
 typedef uint64_t u64a2 __attribute__((aligned(2)));
@@ -338,6 +346,26 @@ OZK_DEV void store_some(void *base, int64_t off, int left, int pleft, uint32_t v
         }
     }
 }
+
+// ... of elements that all exist, or are all padding
+template <typename ST>
+OZK_DEV void store_quad(void *base, int64_t off, bool there, uint32_t v[4]) {
+    // (an absent element's int8 quantisation is zero whatever the scale)
+    if constexpr (sizeof(ST) > 1) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = there ? v[u] : 0u;
+    }
+    Store4<ST>::run(base, off, v);
+}
+
+// The forms of the row and column bodies, chosen on the host (split_form), one
+// to a kernel: as branches of one body they cost every column kernel 15 to 58
+// spilled scalar registers, the small ones up to 16 vector registers as well.
+// ozaki_matmul, us, branches / one to a kernel: 192^3 f64 -> 4 int8 15.1 / 13.8,
+// 448^3 18.0 / 16.7, 16 x 512 x 128 x 512 f32 -> 3 fp16 30.8 / 30.1, 2688 x 448 x
+// 128 f32 -> 2 int8 15.8 / 14.1, 613 x 1492 x 1664 f32 -> 5 bf16 (triangle) 87.4 /
+// 83.9, 14 x 256 x 3724 x 158 f32 -> 3 int8 101.6 / 86.0.
+enum { kExact = 0, kWhole = 1, kAny = 2 };
 
 // The same value afresh: the row's limits, taken at each level through this,
 // are compared there, and not held as one lane mask per store across the levels
@@ -430,11 +458,11 @@ OZK_DEV float row_max(float m, float (*red)[RPB][GW], int buf, int grp, int t) {
 
 // One row per group of 64 * GW lanes.  xrow / srow: the row's first element in X
 // and in the slices; K, Kp: its elements in X and in the slices; off: row of
-// this lane's group unused (its lanes only take part in the barriers).  FULL:
-// the group's lanes hold exactly the row, so nothing is tested; else whole
-// chunks inside K go without tests too.  smax(m, l): maximum of the row at
+// this lane's group unused (its lanes only take part in the barriers).  FORM:
+// kExact tests nothing; kWhole takes K and Kp of whole quads; kAny: whole
+// chunks inside K go without tests.  smax(m, l): maximum of the row at
 // level l from a lane's; put(l, c): stores the scale.
-template <typename XC, typename ST, int G, int NC, bool FULL, typename SMax, typename Put>
+template <typename XC, typename ST, int G, int NC, int FORM, typename SMax, typename Put>
 OZK_DEV void split_row(const SplitParams &p, int64_t xrow, int64_t srow, int K, int Kp, bool off,
                        int t, SMax &&smax, Put &&put) {
     using V = typename In<XC>::V;
@@ -443,8 +471,10 @@ OZK_DEV void split_row(const SplitParams &p, int64_t xrow, int64_t srow, int K, 
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int e0 = (c * G + t) * 4;
-        if (FULL || (c + 1) * G * 4 <= K)
+        if (FORM == kExact || (FORM == kAny && (c + 1) * G * 4 <= K))
             Load<XC>::template vec<4>(p.X, xrow + e0, p.x_code, v + 4 * c);
+        else if (FORM == kWhole)
+            load_quad<XC, 4>(p.X, xrow + e0, e0 < K && !off, p.x_code, v + 4 * c);
         else
             load_some<XC, 4>(p.X, xrow + e0, off ? 0 : K - e0, p.x_code, v + 4 * c);
     }
@@ -462,7 +492,7 @@ OZK_DEV void split_row(const SplitParams &p, int64_t xrow, int64_t srow, int K, 
 #pragma unroll
         for (int ch = 0; ch < NC; ++ch) {
             const int e0 = (ch * G + lt) * 4;
-            if (!FULL && ch * G * 4 >= Kps) {   // a chunk past the row's end
+            if (FORM != kExact && ch * G * 4 >= Kps) {   // a chunk past the row's end
                 if (decltype(first)::value)
 #pragma unroll
                     for (int u = 0; u < 4; ++u) w[ch * 4 + u] = 0.0f;
@@ -471,8 +501,11 @@ OZK_DEV void split_row(const SplitParams &p, int64_t xrow, int64_t srow, int K, 
             uint32_t qv[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) qv[u] = Quant<ST, MODE>::run(src[ch * 4 + u], c, &w[ch * 4 + u]);
-            if (FULL || ((ch + 1) * G * 4 <= Ks && !off)) Store4<ST>::run(p.slices, sl + e0, qv);
-            else if (!off) store_some<ST>(p.slices, sl + e0, Ks - e0, Kps - e0, qv);
+            if (FORM == kExact || (FORM == kAny && (ch + 1) * G * 4 <= Ks && !off))
+                Store4<ST>::run(p.slices, sl + e0, qv);
+            else if (FORM == kWhole) {
+                if (e0 < Kps && !off) store_quad<ST>(p.slices, sl + e0, e0 < Ks, qv);
+            } else if (!off) store_some<ST>(p.slices, sl + e0, Ks - e0, Kps - e0, qv);
             // the residuals here, not at their first use (the next level's
             // maximum): sunk there, every input and every slice value are live
             // at once
@@ -492,7 +525,7 @@ OZK_DEV void split_row(const SplitParams &p, int64_t xrow, int64_t srow, int K, 
 }
 
 // The body of the row kernel for row block `block`; red: LDS for the row maxima.
-template <typename XC, typename ST, int GW, int RPB, int NC>
+template <typename XC, typename ST, int GW, int RPB, int NC, int FORM>
 OZK_DEV void split_rows_body(const SplitParams &p, int64_t block, float (*red)[RPB][GW]) {
     constexpr int G = 64 * GW;
     const int tid = threadIdx.x;
@@ -510,17 +543,13 @@ OZK_DEV void split_rows_body(const SplitParams &p, int64_t block, float (*red)[R
         if (!off && t == 0) srow_scale[l * p.cs_l] = c.s;
     };
     const int64_t xrow = b * p.xs_b + r * p.xs_r, srow = b * p.ss_b + r * p.ss_r;
-    // (uniform over the workgroup: the paths hold barriers)
-    if (p.K == 4 * NC * G && block * RPB + RPB <= nrows)
-        split_row<XC, ST, G, NC, true>(p, xrow, srow, 0, 0, false, t, smax, put);
-    else
-        split_row<XC, ST, G, NC, false>(p, xrow, srow, (int)p.K, (int)p.Kp, off, t, smax, put);
+    split_row<XC, ST, G, NC, FORM>(p, xrow, srow, (int)p.K, (int)p.Kp, off, t, smax, put);
 }
 
-template <typename XC, typename ST, int GW, int RPB, int NC>
+template <typename XC, typename ST, int GW, int RPB, int NC, int FORM>
 __global__ __launch_bounds__(64 * GW * RPB) void split_rows_kernel(SplitParams p) {
     __shared__ float red[2][RPB][GW];
-    split_rows_body<XC, ST, GW, RPB, NC>(p, blockIdx.x, red);
+    split_rows_body<XC, ST, GW, RPB, NC, FORM>(p, blockIdx.x, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -603,11 +632,11 @@ OZK_DEV void cols_scale(float m[VEC], ColsShared<NT, SEG, VEC> &sh, int buf, int
 // column) in X and in the slices; K, Kp: rows from there on, with the padding;
 // ncol: of its VEC columns, those that exist; col_ok, kin: uniform over the
 // workgroup, every lane has VEC columns / rows below kin exist for every lane.
-// FULL: the workgroup holds whole columns of exactly K rows, nothing is tested;
-// SKIP: its rows past the last one are left out.
+// FORM: kExact tests nothing; kWhole: every lane has all of its columns or none,
+// K and Kp are whole quads; SKIP: rows past the last one are left out.
 // scale(m, l, c): the level's constants of the lane's columns from its maxima;
 // put(l, c): stores their scales.
-template <typename XC, typename ST, int RPP, int NQ, bool FULL, bool SKIP, typename Scale,
+template <typename XC, typename ST, int RPP, int NQ, int FORM, bool SKIP, typename Scale,
           typename Put>
 OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, int Kp, int ncol,
                         bool col_ok, int kin, Scale &&scale, Put &&put) {
@@ -619,8 +648,11 @@ OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, 
 #pragma unroll
         for (int dk = 0; dk < 4; ++dk) {
             const int k = 4 * g * RPP + dk;
-            if (FULL || (col_ok && 4 * (g + 1) * RPP <= kin))
+            if (FORM == kExact || (FORM == kAny && col_ok && 4 * (g + 1) * RPP <= kin))
                 Load<XC>::template vec<VEC>(p.X, xb + k * p.xs_k, p.x_code, v[g][dk]);
+            else if (FORM == kWhole)
+                load_quad<XC, VEC>(p.X, xb + k * p.xs_k, 4 * g * RPP < K && ncol > 0, p.x_code,
+                                   v[g][dk]);
             else
                 load_some<XC, VEC>(p.X, xb + k * p.xs_k, k < K ? ncol : 0, p.x_code, v[g][dk]);
         }
@@ -660,10 +692,16 @@ OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, 
 #pragma unroll
                 for (int u = 0; u < VEC; ++u)
                     qv[u][dk] = Quant<ST, MODE>::run(src[g][dk][u], c[u], &w[g][dk][u]);
-            if (FULL || (col_ok && 4 * (g + 1) * RPP <= kin)) {
+            if (FORM == kExact || (FORM == kAny && col_ok && 4 * (g + 1) * RPP <= kin)) {
 #pragma unroll
                 for (int u = 0; u < VEC; ++u)
                     Store4<ST>::run(p.slices, sl + u * p.ss_r + k0, qv[u]);
+            } else if (FORM == kWhole) {
+                if (k0 < Kps && nc > 0) {
+#pragma unroll
+                    for (int u = 0; u < VEC; ++u)
+                        store_quad<ST>(p.slices, sl + u * p.ss_r + k0, k0 < Ks, qv[u]);
+                }
             } else {
 #pragma unroll
                 for (int u = 0; u < VEC; ++u)
@@ -691,7 +729,7 @@ OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, 
     }
 }
 
-template <typename XC, typename ST, int NT, int SEG, int NQ>
+template <typename XC, typename ST, int NT, int SEG, int NQ, int FORM>
 OZK_DEV void split_cols_body(const SplitParams &p, int64_t sidx,
                              ColsShared<NT, SEG, In<XC>::VEC> &sh) {
     constexpr int VEC = In<XC>::VEC;
@@ -715,20 +753,17 @@ OZK_DEV void split_cols_body(const SplitParams &p, int64_t sidx,
         if (ro == 0) {
 #pragma unroll
             for (int u = 0; u < VEC; ++u)
-                if (u < ncol) sc_base[l * p.cs_l + u * p.cs_r] = c[u].s;
+                if (FORM == kExact || u < ncol) sc_base[l * p.cs_l + u * p.cs_r] = c[u].s;
         }
     };
-    if (col_ok && p.K == 4 * NQ * RPP)
-        split_cols<XC, ST, RPP, NQ, true, false>(p, xb, sbase, 0, 0, 0, true, 0, scale, put);
-    else
-        split_cols<XC, ST, RPP, NQ, false, true>(p, xb, sbase, (int)p.K - 4 * ro, (int)p.Kp - 4 * ro,
-                                                 ncol, col_ok, (int)p.K, scale, put);
+    split_cols<XC, ST, RPP, NQ, FORM, FORM != kExact>(
+        p, xb, sbase, (int)p.K - 4 * ro, (int)p.Kp - 4 * ro, ncol, col_ok, (int)p.K, scale, put);
 }
 
-template <typename XC, typename ST, int NT, int SEG, int NQ>
+template <typename XC, typename ST, int NT, int SEG, int NQ, int FORM>
 __global__ __launch_bounds__(NT) void split_cols_kernel(SplitParams p) {
     __shared__ ColsShared<NT, SEG, In<XC>::VEC> sh;
-    split_cols_body<XC, ST, NT, SEG, NQ>(p, xcd_remap(blockIdx.x, (int64_t)gridDim.x), sh);
+    split_cols_body<XC, ST, NT, SEG, NQ, FORM>(p, xcd_remap(blockIdx.x, (int64_t)gridDim.x), sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -739,10 +774,9 @@ __global__ __launch_bounds__(NT) void split_cols_kernel(SplitParams p) {
 struct FusedSplit {
     SplitParams op[2];
 };
-// (SEG = 0: rows only; the smallest column groups at eight waves a SIMD, which
-// their launch's rows need: 16 x 512 x 128 x 512 f32 -> 3 fp16 30.3 us, else 31.2)
-template <typename XC, typename ST, int NT, int GW, int NC, int SEG, int NQ>
-__global__ __launch_bounds__(NT, NQ == 1 ? 8 : 1) void split_fused_kernel(FusedSplit f, int64_t n0) {
+// (SEG = 0: rows only)
+template <typename XC, typename ST, int NT, int GW, int NC, int SEG, int NQ, int FORM>
+__global__ __launch_bounds__(NT) void split_fused_kernel(FusedSplit f, int64_t n0) {
     const int which = (int64_t)blockIdx.x >= n0;
     const SplitParams &p = f.op[which];
     const int64_t g = (int64_t)blockIdx.x - (which ? n0 : 0);
@@ -753,12 +787,12 @@ __global__ __launch_bounds__(NT, NQ == 1 ? 8 : 1) void split_fused_kernel(FusedS
     } sh;
     if constexpr (SEG > 0) {
         if (p.cols) {
-            split_cols_body<XC, ST, NT, SEG, NQ>(
+            split_cols_body<XC, ST, NT, SEG, NQ, FORM>(
                 p, xcd_remap(g, which ? (int64_t)gridDim.x - n0 : n0), sh.cols);
             return;
         }
     }
-    split_rows_body<XC, ST, GW, RPB, NC>(p, g, sh.rows);
+    split_rows_body<XC, ST, GW, RPB, NC, FORM>(p, g, sh.rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -922,9 +956,9 @@ OZK_DEV void split_coop_body(const SplitParams &p, uint64_t *slot, int P, uint32
     };
     auto put = [](int, const LevelScale *) {};
     if (col_ok && kin == 4 * NG * RPP)
-        split_cols<XT, ST, RPP, NG, true, false>(p, xb, sbase, 0, 0, 0, true, 0, scale, put);
+        split_cols<XT, ST, RPP, NG, kExact, false>(p, xb, sbase, 0, 0, 0, true, 0, scale, put);
     else
-        split_cols<XT, ST, RPP, NG, false, false>(p, xb, sbase, K, Kp, ncol, col_ok, kin, scale, put);
+        split_cols<XT, ST, RPP, NG, kAny, false>(p, xb, sbase, K, Kp, ncol, col_ok, kin, scale, put);
 }
 
 template <typename XT, typename ST, int RPL, int SEG>
@@ -962,7 +996,9 @@ __global__ __launch_bounds__(kCoopNT) void split_pair_kernel(SplitParams pb, uin
         split_coop_body<XT, ST, RPL, 8>(pb, slot, P, want_tag, tick_limit, status, q * P + pos, sh);
     } else {
         const int64_t ab = q * ka + (pos - P);
-        if (ab < pa.batch * pa.rows) split_rows_body<XT, ST, 4, 1, NC>(pa, ab, red);
+        if (ab >= pa.batch * pa.rows) return;
+        if (pa.K == 4 * NC * 256) split_rows_body<XT, ST, 4, 1, NC, kExact>(pa, ab, red);
+        else split_rows_body<XT, ST, 4, 1, NC, kAny>(pa, ab, red);
     }
 }
 
@@ -1048,9 +1084,9 @@ __global__ __launch_bounds__(64 * GW) void split_rows_coop_kernel(SplitParams p,
     };
 
     if (kleft >= CHR)
-        split_row<XT, ST, G, NC, true>(p, xrow, srow, 0, 0, false, t, rmax, store_scale);
+        split_row<XT, ST, G, NC, kExact>(p, xrow, srow, 0, 0, false, t, rmax, store_scale);
     else
-        split_row<XT, ST, G, NC, false>(p, xrow, srow, kleft, sleft, false, t, rmax, store_scale);
+        split_row<XT, ST, G, NC, kAny>(p, xrow, srow, kleft, sleft, false, t, rmax, store_scale);
 }
 
 // ---------------------------------------------------------------------------
@@ -1177,30 +1213,49 @@ static hipError_t launch_cols_coop(const SplitParams &p, int seg, hipStream_t st
     return P > 1 ? launch_poison(p, slot + n, st) : hipSuccess;
 }
 
+// The form an operand allows: cap, the K a workgroup's lanes hold exactly; n, the
+// rows or columns of a workgroup; vec, the columns of a lane.
+static int split_form(const SplitParams &p, bool cols, int64_t cap, int64_t n, int64_t vec) {
+    const int64_t total = cols ? p.rows : p.batch * p.rows;
+    if (p.K == cap && total % n == 0) return kExact;
+    return p.K % 4 == 0 && p.Kp % 4 == 0 && (!cols || p.rows % vec == 0) ? kWhole : kAny;
+}
+// f(integral constant) for a form
+template <typename F> static void with_form(int form, F &&f) {
+    if (form == kExact) f(std::integral_constant<int, kExact>{});
+    else if (form == kWhole) f(std::integral_constant<int, kWhole>{});
+    else f(std::integral_constant<int, kAny>{});
+}
+
 // rows and columns longer than the fused kernel takes (variants 6 on)
+template <typename XT, typename ST, int GW, int NC>
+static void launch_long_rows(const SplitParams &p, hipStream_t st) {
+    with_form(split_form(p, false, 4 * NC * 64 * GW, 1, 1), [&](auto form) {
+        hipLaunchKernelGGL((split_rows_kernel<XT, ST, GW, 1, NC, decltype(form)::value>),
+                           dim3((unsigned)(p.batch * p.rows)), dim3(64 * GW), 0, st, p);
+    });
+}
+template <typename XT, typename ST, int NT, int NQ>
+static void launch_long_cols(const SplitParams &p, hipStream_t st) {
+    constexpr int VEC = In<XT>::VEC;
+    with_form(split_form(p, true, 4 * NQ * NT, VEC, VEC), [&](auto form) {
+        hipLaunchKernelGGL((split_cols_kernel<XT, ST, NT, 1, NQ, decltype(form)::value>),
+                           dim3((unsigned)(p.batch * ((p.rows + VEC - 1) / VEC))), dim3(NT), 0, st, p);
+    });
+}
 template <typename XT, typename ST>
 static hipError_t launch_long(const SplitParams &p, const SplitPlan &plan, hipStream_t st) {
-    const int64_t nrows = p.batch * p.rows;
-#define OZK_ROWS(GW, NC)                                                                    \
-    hipLaunchKernelGGL((split_rows_kernel<XT, ST, GW, 1, NC>), dim3((unsigned)nrows),       \
-                       dim3(64 * GW), 0, st, p)
-#define OZK_COLS(NT, NQ)                                                                    \
-    hipLaunchKernelGGL((split_cols_kernel<XT, ST, NT, 1, NQ>),                              \
-                       dim3((unsigned)(p.batch * ((p.rows + In<XT>::VEC - 1) / In<XT>::VEC))), \
-                       dim3(NT), 0, st, p)
-    if (plan.path == kSplitRows && plan.variant == 6) OZK_ROWS(8, 8);
-    else if (plan.path == kSplitRows && plan.variant == 7) OZK_ROWS(16, 8);
+    constexpr bool F32 = sizeof(XT) == 4;
+    if (plan.path == kSplitRows && plan.variant == 6) launch_long_rows<XT, ST, 8, 8>(p, st);
+    else if (plan.path == kSplitRows && plan.variant == 7) launch_long_rows<XT, ST, 16, 8>(p, st);
     else if (plan.path == kSplitRows && plan.variant == 8) {
-        if constexpr (sizeof(XT) == 4) OZK_ROWS(16, 16);
+        if constexpr (F32) launch_long_rows<XT, ST, 16, 16>(p, st);
         else return hipErrorInvalidValue;
     } else if (plan.path == kSplitStrip && plan.variant == 6) {
-        if constexpr (sizeof(XT) == 4) OZK_COLS(1024, 4);
-        else OZK_COLS(512, 8);
+        launch_long_cols<XT, ST, F32 ? 1024 : 512, F32 ? 4 : 8>(p, st);
     } else {
         return hipErrorInvalidValue;
     }
-#undef OZK_ROWS
-#undef OZK_COLS
     return hipGetLastError();
 }
 
@@ -1226,18 +1281,26 @@ static hipError_t launch_long(const SplitParams &p, const SplitPlan &plan, hipSt
 // 4096^2 f32 -> 2 fp16 68 / 66, f64 -> 4 int8 2048 rows and 4096 columns of
 // 2048 41.9 / 39.9, 4096 and 4096 of 1024 27.9 / 24.5 (two launches: 120,
 // 67, 47, 28).
-enum { kNoCols = 0, kNarrowCols = 1, kWideCols = 2 };
 template <typename XC, typename ST, int NT, int GW, int NC, int SEG, int NQ>
 static hipError_t launch_fused_cfg(const FusedSplit &f, int n, hipStream_t st) {
+    constexpr int VEC = In<XC>::VEC, SW = SEG > 0 ? SEG * VEC : 1, RPB = NT / (64 * GW);
+    constexpr int64_t CAP = 4 * NC * 64 * GW;
+    static_assert(SEG == 0 || CAP == 4 * NQ * (NT / (SEG > 0 ? SEG : 1)),
+                  "rows and columns of one class");
     auto blocks = [](const SplitParams &p) -> int64_t {
-        constexpr int SW = SEG > 0 ? SEG * In<XC>::VEC : 1;
-        constexpr int RPB = NT / (64 * GW);
         return p.cols ? p.batch * ((p.rows + SW - 1) / SW) : (p.batch * p.rows + RPB - 1) / RPB;
     };
+    int form = kExact;
+    for (int i = 0; i < n; ++i) {
+        const int fi = split_form(f.op[i], f.op[i].cols, CAP, f.op[i].cols ? SW : RPB, VEC);
+        form = fi > form ? fi : form;
+    }
     const int64_t n0 = blocks(f.op[0]);
     const int64_t total = n0 + (n > 1 ? blocks(f.op[1]) : 0);
-    hipLaunchKernelGGL((split_fused_kernel<XC, ST, NT, GW, NC, SEG, NQ>), dim3((unsigned)total),
-                       dim3(NT), 0, st, f, n0);
+    with_form(form, [&](auto fm) {
+        hipLaunchKernelGGL((split_fused_kernel<XC, ST, NT, GW, NC, SEG, NQ, decltype(fm)::value>),
+                           dim3((unsigned)total), dim3(NT), 0, st, f, n0);
+    });
     return hipGetLastError();
 }
 template <typename XC, typename ST>

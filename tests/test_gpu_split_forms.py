@@ -1,0 +1,62 @@
+"""The three forms of the split kernels (exact sizes, whole quads, any): slices and
+scales bit for bit against the oracle in every class of K, rows and columns,
+and ozaki_matmul's zero padding of whole quads beside a row with an infinite
+entry."""
+import pytest
+import torch
+
+from tests.helpers import assert_bitwise_equal, oracle_split_batched, sample_indices, to_np
+
+pytestmark = pytest.mark.gpu
+
+SDTS = [torch.int8, torch.float16, torch.bfloat16, torch.float32]
+# (rows, K): K at a class's limit with whole groups; whole quads and groups of
+# columns part empty; the same with wide column groups (fp64 from 256 groups of 8
+# columns at K <= 1024, 512 at K <= 2048, fp64 and fp32 256 of 4 and 8 at K <= 4096)
+EXACT = [(16, 256), (16, 512), (8, 1024), (8, 2048), (8, 4096), (8, 8192), (8, 16384)]
+WHOLE = [(20, 100), (12, 300), (36, 516), (12, 1028), (28, 2052), (12, 4100), (8, 8196), (12, 12292)]
+WIDE = [(2048, 1024), (2060, 1020), (2053, 1021), (2049, 700), (4096, 2048), (4108, 2044),
+        (4099, 2045), (4097, 1500), (2048, 4096), (2060, 4092)]
+
+
+@pytest.mark.parametrize("xdt", [torch.float64, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("columns,rows,K", [(False, *s) for s in EXACT + WHOLE] +
+                         [(True, *s) for s in EXACT + WHOLE + WIDE])
+def test_split_forms(oracle, gpu, columns, rows, K, xdt):
+    import ozaki_triton_amd as ozk
+    sdt = SDTS[(rows // 4 + K // 4 + (xdt == torch.float32)) % 4]
+    L, batch = 1 + (rows + K // 4) % 4, 2 if rows * K < 1 << 20 else 1
+    print(f"[forms] {rows}x{K} {xdt} -> {sdt} L={L} columns={columns}", flush=True)
+    g = torch.Generator().manual_seed(rows * 17 + K)
+    X = torch.randn(batch, rows, K, generator=g, dtype=torch.float64)
+    X = (X * torch.pow(2.0, torch.randint(-3, 4, (batch, rows, 1), generator=g).double())).to(xdt)
+    Xd = X.to(gpu)
+    if columns:
+        Xd = Xd.mT.contiguous().mT
+    alpha = ozk.compute_split_bits(K, sdt, torch.int32 if sdt == torch.int8 else torch.float32)
+    sl, sc = ozk.split_matrix(Xd, L, alpha, sdt)
+    torch.cuda.synchronize()
+    idx = sample_indices(rows, min(rows, 24), K)
+    osl, osc = oracle_split_batched(oracle, to_np(X[:, idx].contiguous()), L, alpha, sdt)
+    assert_bitwise_equal(to_np(sc[:, :, idx].contiguous()), osc, "scales")
+    assert_bitwise_equal(to_np(sl[:, :, idx].contiguous()), osl, "slices")
+
+
+@pytest.mark.parametrize("sdt", SDTS)
+@pytest.mark.parametrize("xdt", [torch.float64, torch.float32])
+@pytest.mark.parametrize("M,N,K", [(72, 68, 516), (40, 36, 1028)])
+def test_whole_quads_infinite_entries(gpu, M, N, K, xdt, sdt):
+    """Infinite entries spoil their row and column of C only: the quads of padding
+    after a K of whole quads stay zero, whatever the scale."""
+    import ozaki_triton_amd as ozk
+    g = torch.Generator().manual_seed(K)
+    A = torch.randn(M, K, generator=g, dtype=torch.float64).to(xdt)
+    B = torch.randn(K, N, generator=g, dtype=torch.float64).to(xdt)
+    want = ozk.ozaki_matmul(A.to(gpu), B.to(gpu), 3, sdt)
+    A[9, K - 1] = float("inf")
+    B[0, 5] = float("-inf")
+    got = ozk.ozaki_matmul(A.to(gpu), B.to(gpu), 3, sdt)
+    torch.cuda.synchronize()
+    assert not torch.isfinite(got[9]).any() and not torch.isfinite(got[:, 5]).any()
+    rows, cols = [i for i in range(M) if i != 9], [j for j in range(N) if j != 5]
+    assert_bitwise_equal(to_np(got[rows][:, cols]), to_np(want[rows][:, cols]), "other entries")

@@ -1,0 +1,68 @@
+"""Registers of the split kernels, from the metadata of the built library's code
+objects: no form may spill vector registers, the exact and small ones nothing at
+all (branches for every form in one kernel once spilled 15 to 58 scalar and up
+to 16 vector registers, and products of a few hundred rows were 2-7% slower)."""
+import re
+import shutil
+import struct
+import subprocess
+
+import pytest
+
+READELF = shutil.which("llvm-readelf") or "/opt/rocm/llvm/bin/llvm-readelf"
+
+
+def _code_objects(path):
+    """The gfx code objects of the offload bundles in a library."""
+    data = open(path, "rb").read()
+    magic, at = b"__CLANG_OFFLOAD_BUNDLE__", 0
+    while (at := data.find(magic, at)) >= 0:
+        entries, = struct.unpack_from("<Q", data, at + 24)
+        p = at + 32
+        for _ in range(entries):
+            offset, size, n = struct.unpack_from("<QQQ", data, p)
+            name = data[p + 24:p + 24 + n]
+            p += 24 + n
+            if b"amdgcn" in name and size:
+                yield data[at + offset:at + offset + size]
+        at += len(magic)
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    from ozaki_triton_amd import build
+    if not shutil.which(READELF):
+        pytest.skip("no llvm-readelf")
+    out, tmp = {}, tmp_path_factory.mktemp("co") / "object"
+    for obj in _code_objects(build.LIB_PATH):
+        tmp.write_bytes(obj)
+        notes = subprocess.run([READELF, "--notes", str(tmp)], capture_output=True, text=True).stdout
+        for block in notes.split("  - .agpr_count:")[1:]:
+            f = dict(re.findall(r"\.(name|sgpr_spill_count|vgpr_spill_count|"
+                                r"private_segment_fixed_size):\s+(\S+)", block))
+            out[f["name"]] = tuple(int(f[k]) for k in ("sgpr_spill_count", "vgpr_spill_count",
+                                                       "private_segment_fixed_size"))
+    return out
+
+
+def test_split_kernels_spill_no_vector_registers(kernels):
+    split = {n: r for n, r in kernels.items() if "split_" in n}
+    assert len(split) > 100
+    assert {n: r for n, r in split.items() if r[1] != 0} == {}
+
+
+def test_exact_and_small_forms_spill_nothing(kernels):
+    """The template's last arguments: 16-byte pieces of a row, quads of a lane, form
+    (0 exact, 1 whole quads, 2 any)."""
+    seen = 0
+    for name, (sgpr, vgpr, scratch) in kernels.items():
+        m = re.search(r"18split_fused_kernel.*?Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)EEE", name)
+        if not m:
+            continue
+        seg, nq, form = map(int, m.groups()[3:])
+        seen += 1
+        if form == 0 and seg != 1:      # no columns, or more than one piece a row
+            assert (sgpr, vgpr, scratch) == (0, 0, 0), name
+        if form < 2 and nq <= 1:        # K <= 512, rows alone
+            assert (vgpr, scratch) == (0, 0), name
+    assert seen > 100
