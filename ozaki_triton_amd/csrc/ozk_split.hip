@@ -353,6 +353,27 @@ static SplitPlan converted_plan(const SplitParams &p, const SplitPlan &plan, int
     return plan_split(q, 1, slice_dtype);
 }
 
+// What is transposed at a time: the whole operand, or where it could do without
+// scratch at most kTransposePart bytes (so that such operands, which the generic
+// kernel splits with none, do not take their own size of it): whole batches or
+// rows of one, 64 rows or more.  Split alone, us, parts of 64 / 128 MiB / whole:
+// 900 rows of 33001 f64 -> 1 int8 199 / 176 / 173, 4000 -> 4 1123 / 885 / 889,
+// 1000 of 65535 f32 -> 3 285 / 231 / 243, 3000 of 20001 f32 -> 2 249 / 210 / 231.
+constexpr int64_t kTransposePart = (int64_t)128 << 20;
+static SplitParams transpose_part(const SplitParams &p, int x_dtype, int slice_dtype) {
+    SplitParams q = p;
+    if (p.K == 0 || !scratch_optional(p, x_dtype, slice_dtype)) return q;
+    const int64_t n = kTransposePart / (p.K * dtype_size(x_dtype)) / 64 * 64;
+    const int64_t rows = n > 64 ? n : 64;
+    if (p.rows > rows) {
+        q.batch = 1;
+        q.rows = rows;
+    } else if (p.batch * p.rows > rows) {
+        q.batch = rows / p.rows;
+    }
+    return q;
+}
+
 size_t split_workspace_bytes(const SplitParams &p, const SplitPlan &plan, int x_dtype,
                              int slice_dtype) {
     const int64_t n = p.batch * p.rows * p.K;
@@ -365,9 +386,10 @@ size_t split_workspace_bytes(const SplitParams &p, const SplitPlan &plan, int x_
     // copy stays reserved, for other pointers and forced kernels
     if (x_dtype >= 2) return (size_t)(n * 4);
     if (plan.path == kSplitTransposeRows) {
-        const size_t tb = (size_t)(n * dtype_size(x_dtype));
+        const SplitParams q = transpose_part(p, x_dtype, slice_dtype);
+        const size_t tb = (size_t)(q.batch * q.rows * q.K * dtype_size(x_dtype));
         if (plan.variant != kRowsCoopVariant) return tb;
-        return round256(tb) + rows_coop_slot_bytes(p, dtype_size(x_dtype));
+        return round256(tb) + rows_coop_slot_bytes(q, dtype_size(x_dtype));
     }
     if (plan.path == kSplitRows && plan.variant == kRowsCoopVariant)
         return rows_coop_slot_bytes(p, dtype_size(x_dtype));
@@ -480,18 +502,33 @@ hipError_t launch_split(const SplitParams &p, const SplitPlan &plan, int x_dtype
         return launch_split(q, converted_plan(p, plan, slice_dtype), 1, slice_dtype, st);
     }
     if (plan.path == kSplitTransposeRows) {
-        // workspace: [batch, rows, K], then the shared row kernel's exchange words
-        const hipError_t e = x_dtype == 0 ? launch_transpose<double>(p, (double *)p.resid, st)
-                                          : launch_transpose<float>(p, p.resid, st);
-        if (e != hipSuccess) return e;
-        SplitParams q = p;
-        q.X = p.resid;
-        q.xs_b = p.rows * p.K;
-        q.xs_r = p.K;
-        q.xs_k = 1;
-        const size_t tb = (size_t)(p.batch * p.rows * p.K) * dtype_size(x_dtype);
-        q.resid = (float *)((char *)p.resid + round256(tb));
-        return launch_split(q, {kSplitRows, plan.variant}, x_dtype, slice_dtype, st);
+        // workspace: [batch, rows, K] of a part, then the shared row kernel's
+        // exchange words
+        const SplitParams part = transpose_part(p, x_dtype, slice_dtype);
+        const int xsz = dtype_size(x_dtype), ssz = dtype_size(slice_dtype);
+        const size_t tb = (size_t)(part.batch * part.rows * p.K) * xsz;
+        for (int64_t b = 0; b < p.batch; b += part.batch)
+            for (int64_t r = 0; r < p.rows; r += part.rows) {
+                SplitParams q = p;
+                q.batch = p.batch - b < part.batch ? p.batch - b : part.batch;
+                q.rows = p.rows - r < part.rows ? p.rows - r : part.rows;
+                q.X = (const char *)p.X + (b * p.xs_b + r * p.xs_r) * xsz;
+                q.slices = (char *)p.slices + (b * p.ss_b + r * p.ss_r) * ssz;
+                q.scales = p.scales + b * p.cs_b + r * p.cs_r;
+                // the parts share one status word: each checks its own
+                if (q.batch != p.batch || q.rows != p.rows) q.fail_out = nullptr;
+                hipError_t e = x_dtype == 0 ? launch_transpose<double>(q, (double *)p.resid, st)
+                                            : launch_transpose<float>(q, p.resid, st);
+                if (e != hipSuccess) return e;
+                q.X = p.resid;
+                q.xs_b = q.rows * q.K;
+                q.xs_r = q.K;
+                q.xs_k = 1;
+                q.resid = (float *)((char *)p.resid + round256(tb));
+                e = launch_split(q, {kSplitRows, plan.variant}, x_dtype, slice_dtype, st);
+                if (e != hipSuccess) return e;
+            }
+        return hipSuccess;
     }
     return with_slice(slice_dtype, [&](auto s) { return s.one(p, plan, x_dtype, st); });
 }

@@ -1,7 +1,8 @@
 """Long operands that are not whole 16-byte pieces (K % 4, pitch, alignment) with
 less scratch than their plan would take: they run on the generic split kernel,
 in ozk_matmul_static's 64 MiB and without a workspace in ozk_split; whole
-operands are refused there."""
+operands are refused there.  And with all they ask for: long columns are
+transposed in parts of 128 MiB."""
 import ctypes
 
 import pytest
@@ -97,3 +98,56 @@ def test_split_without_a_workspace(oracle, gpu, columns, rows, K, xdt):
         osl, osc = oracle_split_batched(oracle, to_np(X), L, alpha, torch.int8)
         assert_bitwise_equal(to_np(sc), osc, "scales")
         assert_bitwise_equal(to_np(sl), osl, "slices")
+
+
+# batch, rows (columns of the operand in memory), K, dtype: several parts of
+# 128 MiB, of one batch's rows (the last part short) and of whole batches
+PARTS = [(1, 1100, 33001, "float64"), (2, 513, 33003, "float64"), (37, 100, 16387, "float32")]
+
+
+def _split_bytes(lib, batch, rows, K, xdt, L):
+    from ozaki_triton_amd import _lib
+    nb = ctypes.c_size_t(0)
+    st = lib.ozk_split_workspace_bytes(
+        _lib.OZK_F64 if xdt == "float64" else _lib.OZK_F32, batch, rows, K,
+        _lib.i64arr([rows * K, 1, rows]), L, _lib.OZK_I8,
+        _lib.i64arr([L * rows * K, rows * K, K, 1]), ctypes.byref(nb))
+    assert st == 0
+    return nb.value
+
+
+@pytest.mark.parametrize("batch,rows,K,xdt", PARTS + [(4, 16384, 65537, "float64")])
+def test_transposed_parts_are_bounded(batch, rows, K, xdt):
+    from ozaki_triton_amd import _lib
+    got = _split_bytes(_lib.load(), batch, rows, K, xdt, 1)
+    assert 64 << 20 < got <= 130 << 20 < batch * rows * K * (8 if xdt == "float64" else 4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,rows,K,xdt", PARTS)
+def test_split_transposed_in_parts(oracle, gpu, force, batch, rows, K, xdt):
+    import ozaki_triton_amd as ozk
+    from ozaki_triton_amd import _lib
+    L, alpha = 2, 7
+    print(f"[parts] {batch}x{rows}x{K} {xdt}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(K)
+    Xd = torch.randn(batch, K, rows, generator=g, dtype=getattr(torch, xdt), device=gpu).mT
+    sl, sc = ozk.split_matrix(Xd, L, alpha, torch.int8)
+    force(split="generic")
+    gsl, gsc = ozk.split_matrix(Xd, L, alpha, torch.int8)
+    torch.cuda.synchronize()
+    assert torch.equal(sc, gsc) and torch.equal(sl, gsl)
+    for b in (0, batch - 1):
+        idx = torch.tensor([0, rows // 2, rows - 1], device=gpu)
+        osl, osc = oracle_split_batched(oracle, to_np(Xd[b:b + 1, idx].contiguous()), L, alpha,
+                                        torch.int8)
+        assert_bitwise_equal(to_np(sc[b:b + 1, :, idx].contiguous()), osc, "scales")
+        assert_bitwise_equal(to_np(sl[b:b + 1, :, idx].contiguous()), osl, "slices")
+    # waits that give up: every part's scales are NaN, the device status is set
+    force(split="", coop_timeout=True)
+    ozk.device_status()
+    sl, sc = ozk.split_matrix(Xd, L, alpha, torch.int8)
+    torch.cuda.synchronize()
+    assert torch.isnan(sc).all()
+    with pytest.raises(_lib.OzakiLibError):
+        ozk.device_status()
