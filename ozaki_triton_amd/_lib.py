@@ -54,6 +54,7 @@ EXPORTED_DEBUG = (
     "ozk_debug_coop_residency",
     "ozk_debug_gemm_kernel",
     "ozk_debug_gemm_kernel_pairs",
+    "ozk_debug_gemm_kernel_out",
     "ozk_debug_split_kernel",
     "ozk_debug_matmul_workspace",
 )
@@ -134,6 +135,10 @@ def load() -> ctypes.CDLL:
                                               ctypes.POINTER(ctypes.c_char_p),
                                               ctypes.POINTER(ctypes.c_int)]
     L.ozk_debug_gemm_kernel_pairs.restype = i32
+    L.ozk_debug_gemm_kernel_out.argtypes = [i64, i64, i64, i64, i32, i32, i32, i32, i32,
+                                            ctypes.POINTER(ctypes.c_char_p),
+                                            ctypes.POINTER(ctypes.c_int)]
+    L.ozk_debug_gemm_kernel_out.restype = i32
     L.ozk_debug_split_kernel.argtypes = [vp, i32, i64, i64, i64, p64, i32, i32, vp, p64,
                                          ctypes.POINTER(ctypes.c_char_p), ctypes.POINTER(sz)]
     L.ozk_debug_split_kernel.restype = i32

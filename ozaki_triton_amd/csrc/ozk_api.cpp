@@ -742,8 +742,15 @@ int ozk_debug_gemm_kernel(int64_t batch, int64_t M, int64_t N, int64_t K, int nu
 int ozk_debug_gemm_kernel_pairs(int64_t batch, int64_t M, int64_t N, int64_t K, int num_splits,
                                 int slice_dtype, int pairs, int cus, const char **name_out,
                                 int *ksplit_out) {
+    return ozk_debug_gemm_kernel_out(batch, M, N, K, num_splits, slice_dtype, pairs, OZK_F64, cus,
+                                     name_out, ksplit_out);
+}
+
+int ozk_debug_gemm_kernel_out(int64_t batch, int64_t M, int64_t N, int64_t K, int num_splits,
+                              int slice_dtype, int pairs, int out_dtype, int cus,
+                              const char **name_out, int *ksplit_out) {
     if (!name_out) return OZK_ERR_NULL;
-    if (!is_slice_dtype(slice_dtype)) return OZK_ERR_DTYPE;
+    if (!is_slice_dtype(slice_dtype) || !is_input_dtype(out_dtype)) return OZK_ERR_DTYPE;
     if (num_splits < 1 || num_splits > OZK_MAX_SPLITS || !pair_set_ok(pairs, num_splits))
         return OZK_ERR_SPLITS;
     if (batch < 0 || M < 0 || N < 0 || K < 0) return OZK_ERR_SHAPE;
@@ -761,7 +768,7 @@ int ozk_debug_gemm_kernel_pairs(int64_t batch, int64_t M, int64_t N, int64_t K, 
     p.M = M;
     p.N = N;
     p.K = K;
-    p.out_dtype = OZK_F64;
+    p.out_dtype = out_dtype;
     p.tri = pairs == OZK_PAIRS_TRIANGULAR && num_splits >= 2;
     const ozk::GemmPlan plan = ozk::plan_gemm(p, num_splits, slice_dtype, cus);
     *name_out = name_of(kGemmNames, plan.kind);

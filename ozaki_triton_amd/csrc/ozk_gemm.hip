@@ -302,8 +302,13 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
     // row of K, in bytes, and on grids that occupy the CUs.  Cross-GEMM alone
     // (kernel trace), the other kernel's time over this one's, int8 into fp64
     // by bytes of K, in brackets fp16 into fp32 at as many bytes:
-    //   1 slice, from 512 tiles, any K: 4096^2 128 bytes 2.1 (2.7), 4096 1.6
-    //     (1.7); 2048^2, 256 tiles, 1024 1.00 (0.94), 2048 0.95 (0.86)
+    //   1 slice, from 512 tiles: 4096^2 128 bytes 2.1 (2.7), 4096 1.30 (1.36),
+    //     16384 1.18 (1.20), 65536 1.18 (1.18); 2900^2 4096 1.70 (1.38), 65536
+    //     1.88 (1.42); 2048^2, 256 tiles, 1024 1.00 (0.94), 2048 0.95 (0.86).
+    //     Up to 16384 bytes where the tiles are one round and C is not fp64,
+    //     when the LDS-DMA kernel's are one too: 4096 x 2048, int8 into fp32,
+    //     1024 1.28, 4096 1.02, 16384 1.04, 24576 0.97, 65536 0.87 (1.19, 1.09,
+    //     1.03, 0.93, 0.88; into fp64 1.18 to 1.40 over 4096 to 131072)
     //   2 slices, from 256 tiles, to 1024 bytes: 4096^2 64 1.44 (1.50), 1024
     //     1.10 (1.17), 4096 0.93; 1536^2, 288 tiles, 1.48 to 1.15 (1.37 to
     //     1.15); 1024 x 1536, 192 tiles, 1.08 to 0.95 (0.94 to 0.84)
@@ -328,7 +333,8 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
     const bool short_has = fits && slice_dtype != 1 && (p.tri ? L <= 5 : L <= 4 && L != 3);
     const bool short_kernel =
         short_has && !kstep &&
-        (L == 1   ? short_tiles >= 2 * kCUs
+        (L == 1   ? short_tiles > 2 * kCUs ||
+                      (short_tiles == 2 * kCUs && (p.out_dtype == 0 || kbytes <= 16384))
          : L == 2 ? short_tiles >= kCUs && kbytes <= (p.tri ? 4096 : 1024)
                   : kbytes <= (L == 4 && p.tri && short_tiles > 2 * kCUs ? 1024 : 512));
     if (short_kernel) plan.kind = kGemmShort;
@@ -415,6 +421,8 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
     else if (fits && forced(kGemmKStep2) && L >= 2) plan.kind = kGemmKStep2;
     else if (fits && forced(kGemmSolo) && L == 4 && slice_dtype != 1) plan.kind = kGemmSolo;
     else if (forced(kGemmShort) && short_has) plan.kind = kGemmShort;
+    // (grids of 512 tiles of 128 x 256 take the short-K kernel; fp32 slices do not)
+    if (plan.kind == kGemmDMA && L <= 1 && slice_dtype != 1 && plan.ni == 4) plan.ni = 2;
     // 96 x 64 tiles: groups of 4 tile rows (C3: 7.12-7.16 ms against 7.21-7.23
     // with 8, 7.33-7.35 with 16; cross-GEMM alone, one box)
     if (plan.kind == kGemmWide4) plan.group_m = 4;

@@ -4068,13 +4068,13 @@ __global__ __launch_bounds__(256, 1) void cross_gemm_soloq_kernel(GemmParams p, 
 // leaves the matrix cores idle meanwhile.  Here a second workgroup runs its K
 // loop under the first one's epilogue and loads.  Tiles, by num_splits: 128 x
 // 128 (1), 128 x 64 (2), 64 x 64 (3, triangle), 64 x 32 (4, and 5 on the
-// triangle), a 2 x 2 grid of waves, each wave every pair of its block: at most 144 accumulator
-// registers of the 256 a wave has at two waves per SIMD, and one stage of 128
-// bytes of K (32 to 60 KB).  The
-// stage is not double-buffered: the other workgroup fills the wait.  Fragments,
-// swizzle and MFMAs as in cross_gemm_wideq_kernel, the epilogue tile by tile
-// (16 x 16), in the reference's order.  Smaller tiles move more bytes per MFMA,
-// so longer contractions keep the kernels above (plan_gemm).
+// triangle), a 2 x 2 grid of waves, each wave every pair of its block: at most
+// 128 accumulator registers of the 256 a wave has at two waves per SIMD, and
+// one stage of 128 bytes of K (32 to 60 KB).  The stage is not
+// double-buffered: the other workgroup fills the wait.  Fragments, swizzle and
+// MFMAs as in cross_gemm_wideq_kernel, the epilogue tile by tile (16 x 16), in
+// the reference's order.  Smaller tiles move more bytes per MFMA, so with two
+// slices or more longer contractions keep the kernels above (plan_gemm).
 // ---------------------------------------------------------------------------
 template <int L_> struct ShortShape {
     static constexpr int L = L_;
@@ -4499,7 +4499,11 @@ static hipError_t launch_one(const GemmParams &p, const GemmPlan &plan, hipStrea
     if constexpr (L == 3) {
         if (plan.kind == kGemmWide) return launch_wide<ST, AccT, TRI>(p, plan, st);
     }
-    if (plan.kind == kGemmDMA) return launch_dma<ST, L, MI, NI, AccT, TRI>(p, plan, st);
+    if constexpr (NI < 4 || std::is_same_v<ST, float>) {
+        if (plan.kind == kGemmDMA) return launch_dma<ST, L, MI, NI, AccT, TRI>(p, plan, st);
+    } else {
+        if (plan.kind == kGemmDMA) return hipErrorInvalidValue;   // no plan gives it
+    }
     using Sh = GemmShape<L, MI, NI>;
     auto kern = cross_gemm_kernel<ST, L, MI, NI, AccT, TRI>;
     static std::atomic<uint64_t> lds_set{0};   // devices whose LDS limit is raised

@@ -170,8 +170,8 @@ enum GemmKind {
     kGemmKStep = 8,   // num_splits 1-4 on small grids: 32 x 32 tiles, 4 waves, wave w takes
                       // K step w of every stage and all pairs; summed through the LDS
     kGemmKStep2 = 9,  // the same with 8 waves: two pair groups, two waves per SIMD (L = 2..4)
-    kGemmShort = 10   // num_splits 1-4, a few stages of K: two workgroups of 4 waves per CU, each
-                      // wave every pair of its block
+    kGemmShort = 10   // num_splits 1, 2 and 4, and 2 to 5 on the triangle, a few stages of K (1:
+                      // any): two workgroups of 4 waves per CU, each wave every pair of its block
 };
 struct GemmPlan {
     int mi, ni;       // 2 x 2 kernels: wave tile = (32*mi) x (32*ni)

@@ -1298,27 +1298,40 @@ def test_more_splits_unsupported_combination_raises(gpu):
 
 
 @pytest.mark.parametrize("sdt", [torch.int8, torch.float16])
-@pytest.mark.parametrize("L,batch,M,N", [
-    (1, 1, 4096, 4096),    # 128 x 256 tiles kept (512 of them)
-    (1, 1, 2048, 4096),    # shrunk to 128 x 128
-    (1, 2, 2048, 1024),    # shrunk to 64 x 128 (the reference's published (2, 2048, 1024, 256))
-    (1, 1, 2048, 2048),    # 64 x 128
-    (2, 1, 2048, 2048),    # L = 2: the ring kernel's 128 x 128 tiles (256 of them)
-    (2, 1, 1024, 1024),    # L = 2: 64 x 64 (LDS-DMA kernel)
-    (3, 1, 2048, 2048),    # L = 3: the wide kernel's 64 x 128 tiles (512 of them)
-    (3, 1, 1280, 1280),    # L = 3: wide (200 tiles, one round against the ring's two)
-    (3, 1, 1536, 1536),    # L = 3: ring (288 wide tiles take two rounds, 576 ring tiles three)
-    (3, 2, 1024, 1000),    # L = 3: wide, batch 2, N cutting a tile
+@pytest.mark.parametrize("L,batch,M,N,K,kernel,forced", [
+    (1, 1, 4096, 4096, 256, "short", ""),     # 1024 tiles of 128 x 128
+    (1, 1, 4096, 4096, 256, "dma", "dma"),    # ... 128 x 128
+    (1, 1, 2048, 4096, 256, "short", ""),     # 512 of them
+    (1, 1, 2048, 4096, 256, "dma", "dma"),    # ... 128 x 128
+    (1, 2, 2048, 1024, 256, "dma", ""),   # 64 x 128 (the reference's published (2, 2048, 1024, 256))
+    (1, 1, 2048, 2048, 256, "dma", ""),       # 64 x 128
+    (2, 1, 2048, 2048, 256, "short", ""),     # L = 2: 512 tiles of 128 x 64
+    (2, 1, 2048, 2048, 2048, "ring", ""),     # ... over more K: 128 x 128 (256 of them)
+    (2, 1, 1024, 1024, 256, "dma", ""),       # L = 2: 64 x 64
+    (3, 1, 2048, 2048, 256, "wide", ""),      # L = 3: 64 x 128 tiles (512 of them)
+    (3, 1, 1280, 1280, 256, "wide", ""),      # L = 3: 200 tiles, one round against the ring's two
+    (3, 1, 1536, 1536, 256, "wide", ""),      # L = 3: 288 tiles, two rounds against the ring's three
+    (3, 1, 1024, 1024, 256, "ring", ""),      # L = 3: one round of either
+    (3, 2, 1024, 1000, 256, "wide", ""),      # L = 3: batch 2, N cutting a tile
 ])
-def test_tile_table_shrink_steps(oracle, gpu, sdt, L, batch, M, N):
+def test_tile_table_shrink_steps(oracle, gpu, force, sdt, L, batch, M, N, K, kernel, forced):
     """The tile table (plan_gemm) shrinks 128 x 256 tiles for grids under 512
     workgroups, N first while it is the larger side: every (rows, columns)
     step it can stop at has a kernel.  (An earlier order stopped at 128 x 64,
     which no kernel took: the launch failed.)  At num_splits 3 it takes the
     wide kernel where its rounds of 256 tiles finish sooner than the ring
-    kernel's.  Sampled blocks against the oracle, K = 256."""
+    kernel's.  Each case runs the kernel it names; sampled blocks against the
+    oracle."""
+    import ctypes
     import ozaki_triton_amd as ozk
-    K = 256
+    from ozaki_triton_amd import _lib
+    if forced:
+        force(gemm=forced)
+    name, ks = ctypes.c_char_p(), ctypes.c_int()
+    assert _lib.load().ozk_debug_gemm_kernel_out(
+        batch, M, N, K, L, {torch.int8: _lib.OZK_I8, torch.float16: _lib.OZK_F16}[sdt], 0,
+        _lib.OZK_F32, 0, ctypes.byref(name), ctypes.byref(ks)) == 0
+    assert name.value.decode() == kernel
     A, B = c3_like((batch, M, K), (batch, K, N), seed=M + N + L, dtype=torch.float32)
     C = ozk.ozaki_matmul(A.to(gpu), B.to(gpu), L, sdt)
     torch.cuda.synchronize()

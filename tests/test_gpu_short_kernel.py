@@ -59,3 +59,27 @@ def test_planner_takes_the_short_kernel(gpu, L, pairs, M, N, sdt):
     with _lib.forced_kernels(gemm="solo" if L == 5 else "dma"):
         want = ozk.cross_gemm(*args, torch.float64, pairs=pairs)
     assert_bitwise_equal(to_np(got), to_np(want), f"L{L} {pairs} {sdt}")
+
+
+@pytest.mark.parametrize("sdt", [torch.int8, torch.float16, torch.bfloat16])
+def test_one_slice_long_k(gpu, sdt):
+    """One round of 128 x 128 tiles over more than 16 KB of K into fp32: the LDS-DMA
+    kernel, C bit for bit that of the short-K kernel."""
+    import ozaki_triton_amd as ozk
+    from ozaki_triton_amd import _lib
+    M, N, K = 4000, 2000, 16385 if sdt == torch.int8 else 8200
+    g = torch.Generator(device=gpu).manual_seed(K)
+    A = torch.randint(-32, 33, (1, 1, M, K), generator=g, device=gpu).to(sdt)
+    B = torch.randint(-32, 33, (1, 1, N, K), generator=g, device=gpu).to(sdt)
+    sa, sb = torch.full((1, 1, M), 0.5, device=gpu), torch.full((1, 1, N), 2.0, device=gpu)
+    kind, ks = ctypes.c_char_p(), ctypes.c_int()
+    assert _lib.load().ozk_debug_gemm_kernel_out(
+        1, M, N, K, 1, {torch.int8: _lib.OZK_I8, torch.float16: _lib.OZK_F16,
+                        torch.bfloat16: _lib.OZK_BF16}[sdt], 0, _lib.OZK_F32, 0,
+        ctypes.byref(kind), ctypes.byref(ks)) == 0
+    assert kind.value == b"dma"
+    args = (A, B.transpose(-1, -2), sa, sb, 1, torch.float32)
+    got = ozk.cross_gemm(*args)
+    with _lib.forced_kernels(gemm="short"):
+        want = ozk.cross_gemm(*args)
+    assert_bitwise_equal(to_np(got), to_np(want), str(sdt))
