@@ -899,24 +899,21 @@ def test_ring_kernel_dtypes(oracle, gpu, L, sdt, out, force):
 
 @pytest.mark.parametrize("sdt", [torch.int8, torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("xdt", [torch.float64, torch.float32])
-@pytest.mark.parametrize("a_shape,b_shape", [((2, 96, 200), (2, 200, 72)),    # strip 0, rows 0
-                                             ((40, 400), (400, 136)),         # strip 0, rows 1
-                                             ((3, 50, 1000), (1000, 24)),     # strip 0, rows 2
-                                             ((64, 2000), (2000, 48)),        # strip 1, rows 3
-                                             ((33, 4000), (4000, 40)),        # strip 2, rows 4
-                                             ((20, 8000), (8000, 16))])       # strip 3, rows 5
-def test_split_duo_one_launch(oracle, gpu, sdt, xdt, a_shape, b_shape, force):
-    """ozaki_matmul's two splits in one launch (split_duo_kernel: B's columns
-    by the 256-lane strip kernel, A's rows by a 256-lane row configuration,
-    the strips first): the library records the B phase's two events at one
+@pytest.mark.parametrize("a_shape,b_shape", [((2, 96, 200), (2, 200, 72)),    # K <= 256
+                                             ((40, 400), (400, 136)),         # K <= 512
+                                             ((3, 50, 1000), (1000, 24)),     # K <= 1024
+                                             ((64, 2000), (2000, 48)),        # K <= 2048
+                                             ((33, 4000), (4000, 40)),        # K <= 4096
+                                             ((20, 8000), (8000, 16))])       # K <= 8192
+def test_split_fused_one_launch(oracle, gpu, sdt, xdt, a_shape, b_shape, force):
+    """ozaki_matmul's two splits in one launch (split_fused_kernel: B's columns,
+    then A's rows): the library records the B phase's two events at one
     point; C equals the two-launch pipeline's (a forced split kernel turns
     the single launch off) bit for bit, and the oracle's on sampled blocks
-    (int8 bit-exact, float slices within the fp32 accumulation bound).  The
-    pairs of configurations follow K; the last (K <= 8192) is fp64 only."""
+    (int8 bit-exact, float slices within the fp32 accumulation bound).  One
+    case for each class of K."""
     import ozaki_triton_amd as ozk
     from ozaki_triton_amd.ozaki import _ozaki_matmul_impl
-    if xdt == torch.float32 and a_shape[-1] > 4096:
-        pytest.skip("fp32 columns over 4096 take the 512-lane strip kernel")
     A, B = c3_like(a_shape, b_shape, seed=sum(a_shape) + sum(b_shape) + 7, dtype=xdt)
     Ad, Bd = A.to(gpu), B.to(gpu)
     L = 3
@@ -938,7 +935,7 @@ def test_split_duo_one_launch(oracle, gpu, sdt, xdt, a_shape, b_shape, force):
         Ab = A_np[b] if A_np.ndim == 3 else A_np
         Bb = B_np[b] if B_np.ndim == 3 else B_np
         check_block_vs_oracle(oracle, ozk, Cb, Ab, Bb, rows, cols, L, sdt, xdt,
-                              f"duo {xdt} {sdt} {a_shape} b{b}")
+                              f"fused {xdt} {sdt} {a_shape} b{b}")
 
 
 @pytest.mark.parametrize("xdt", [torch.float64, torch.float32])
