@@ -330,7 +330,10 @@ GemmPlan plan_gemm(const GemmParams &p, int L, int slice_dtype, int cus) {
     const int64_t short_bm = L <= 2 ? 128 : 64, short_bn = L == 1 ? 128 : L <= 3 ? 64 : 32;
     const int64_t short_tiles =
         p.batch * ((p.M + short_bm - 1) / short_bm) * ((p.N + short_bn - 1) / short_bn);
-    const bool short_has = fits && slice_dtype != 1 && (p.tri ? L <= 5 : L <= 4 && L != 3);
+    // (a launch counts its work-items in 32 bits: 256 for 64 x 32 values of C at
+    // most, where wide4 has 512 for 96 x 64)
+    const bool short_has = fits && slice_dtype != 1 && (p.tri ? L <= 5 : L <= 4 && L != 3) &&
+                           short_tiles < (int64_t)1 << 24;
     const bool short_kernel =
         short_has && !kstep &&
         (L == 1   ? short_tiles > 2 * kCUs ||

@@ -1,5 +1,6 @@
 """Where the planner leaves the short-K cross-GEMM kernel (no GPU needed): one
-slice over a long K where both kernels' tiles are one round."""
+slice over a long K where both kernels' tiles are one round, and more tiles
+than one launch counts."""
 import ctypes
 
 import pytest
@@ -28,3 +29,11 @@ def test_one_slice_over_a_long_k(sd, size):
     for M, N in ((4096, 2176), (3000, 3400), (4096, 4096)):
         assert _plan(M, N, 65536 // size, 1, sd, out="float32") == "short"
     assert _plan(2048, 2048, 256, 1, sd, out="float32") == "dma"
+
+
+def test_more_tiles_than_a_launch_counts():
+    """2^24 tiles of 64 x 32 are 2^32 work-items: larger tiles, which launch."""
+    assert _plan(1 << 18, (1 << 17) - 32, 64, 4, "int8") == "short"
+    assert _plan(1 << 18, 1 << 17, 64, 4, "int8") == "wide4"
+    assert _plan(1 << 18, 1 << 17, 64, 5, "int8", "triangular") == "solo"
+    assert _plan(1 << 18, 1 << 17, 64, 4, "float16", "triangular") != "short"
