@@ -477,9 +477,42 @@ static hipError_t launch_convert(const SplitParams &p, float *T, hipStream_t st)
     return hipGetLastError();
 }
 
+// f on parts of an operand, `batch` batches of `rows` rows each or fewer.
+template <typename F>
+static hipError_t for_parts(const SplitParams &p, int64_t batch, int64_t rows, int x_dtype,
+                            int slice_dtype, F &&f) {
+    const int xsz = dtype_size(x_dtype), ssz = dtype_size(slice_dtype);
+    for (int64_t b = 0; b < p.batch; b += batch)
+        for (int64_t r = 0; r < p.rows; r += rows) {
+            SplitParams q = p;
+            q.batch = p.batch - b < batch ? p.batch - b : batch;
+            q.rows = p.rows - r < rows ? p.rows - r : rows;
+            q.X = (const char *)p.X + (b * p.xs_b + r * p.xs_r) * xsz;
+            q.slices = (char *)p.slices + (b * p.ss_b + r * p.ss_r) * ssz;
+            q.scales = p.scales + b * p.cs_b + r * p.cs_r;
+            // the parts share one status word: each checks its own
+            if (q.batch != p.batch || q.rows != p.rows) q.fail_out = nullptr;
+            if (hipError_t e = f(q)) return e;
+        }
+    return hipSuccess;
+}
+
+// A launch counts its work-items in 32 bits, and split_fused_kernel takes up to
+// 256 for a row: the rows of one launch, beside columns.
+constexpr int64_t kFusedRows = (int64_t)1 << 23;
+static bool fused_in_one(const SplitParams &p, const SplitPlan &plan) {
+    return plan.path != kSplitRows || p.batch * p.rows <= kFusedRows;
+}
+
 hipError_t launch_split(const SplitParams &p, const SplitPlan &plan, int x_dtype,
                         int slice_dtype, hipStream_t st) {
     if (p.batch * p.rows == 0 || p.L == 0) return hipSuccess;
+    if (fused_plan(plan) && !fused_in_one(p, plan)) {
+        const int64_t rows = p.rows < kFusedRows ? p.rows : kFusedRows;
+        return for_parts(p, kFusedRows / rows, rows, x_dtype, slice_dtype, [&](const SplitParams &q) {
+            return launch_split(q, plan, x_dtype, slice_dtype, st);
+        });
+    }
     if (fused_plan(plan)) {
         const SplitParams q = fused_params(p, plan, x_dtype);
         return with_slice(slice_dtype, [&](auto s) {
@@ -505,30 +538,19 @@ hipError_t launch_split(const SplitParams &p, const SplitPlan &plan, int x_dtype
         // workspace: [batch, rows, K] of a part, then the shared row kernel's
         // exchange words
         const SplitParams part = transpose_part(p, x_dtype, slice_dtype);
-        const int xsz = dtype_size(x_dtype), ssz = dtype_size(slice_dtype);
+        const int xsz = dtype_size(x_dtype);
         const size_t tb = (size_t)(part.batch * part.rows * p.K) * xsz;
-        for (int64_t b = 0; b < p.batch; b += part.batch)
-            for (int64_t r = 0; r < p.rows; r += part.rows) {
-                SplitParams q = p;
-                q.batch = p.batch - b < part.batch ? p.batch - b : part.batch;
-                q.rows = p.rows - r < part.rows ? p.rows - r : part.rows;
-                q.X = (const char *)p.X + (b * p.xs_b + r * p.xs_r) * xsz;
-                q.slices = (char *)p.slices + (b * p.ss_b + r * p.ss_r) * ssz;
-                q.scales = p.scales + b * p.cs_b + r * p.cs_r;
-                // the parts share one status word: each checks its own
-                if (q.batch != p.batch || q.rows != p.rows) q.fail_out = nullptr;
-                hipError_t e = x_dtype == 0 ? launch_transpose<double>(q, (double *)p.resid, st)
-                                            : launch_transpose<float>(q, p.resid, st);
-                if (e != hipSuccess) return e;
-                q.X = p.resid;
-                q.xs_b = q.rows * q.K;
-                q.xs_r = q.K;
-                q.xs_k = 1;
-                q.resid = (float *)((char *)p.resid + round256(tb));
-                e = launch_split(q, {kSplitRows, plan.variant}, x_dtype, slice_dtype, st);
-                if (e != hipSuccess) return e;
-            }
-        return hipSuccess;
+        return for_parts(p, part.batch, part.rows, x_dtype, slice_dtype, [&](SplitParams q) {
+            const hipError_t e = x_dtype == 0 ? launch_transpose<double>(q, (double *)p.resid, st)
+                                              : launch_transpose<float>(q, p.resid, st);
+            if (e != hipSuccess) return e;
+            q.X = p.resid;
+            q.xs_b = q.rows * q.K;
+            q.xs_r = q.K;
+            q.xs_k = 1;
+            q.resid = (float *)((char *)p.resid + round256(tb));
+            return launch_split(q, {kSplitRows, plan.variant}, x_dtype, slice_dtype, st);
+        });
     }
     return with_slice(slice_dtype, [&](auto s) { return s.one(p, plan, x_dtype, st); });
 }
@@ -556,6 +578,10 @@ hipError_t launch_split_fused(const SplitParams &pa, const SplitPlan &plan_a, co
                               hipStream_t st) {
     if (!split_fused_ok(plan_a, plan_b)) return hipErrorInvalidValue;
     if (pa.batch * pa.rows == 0 || pb.batch * pb.rows == 0 || pa.L == 0) return hipSuccess;
+    if (!fused_in_one(pa, plan_a) || !fused_in_one(pb, plan_b)) {
+        if (hipError_t e = launch_split(pb, plan_b, x_dtype, slice_dtype, st)) return e;
+        return launch_split(pa, plan_a, x_dtype, slice_dtype, st);
+    }
     const SplitParams qa = fused_params(pa, plan_a, x_dtype), qb = fused_params(pb, plan_b, x_dtype);
     const int wa = fused_width(qa, plan_a.variant, x_dtype);
     const int wb = fused_width(qb, plan_b.variant, x_dtype);

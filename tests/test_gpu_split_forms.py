@@ -60,3 +60,23 @@ def test_whole_quads_infinite_entries(gpu, M, N, K, xdt, sdt):
     assert not torch.isfinite(got[9]).any() and not torch.isfinite(got[:, 5]).any()
     rows, cols = [i for i in range(M) if i != 9], [j for j in range(N) if j != 5]
     assert_bitwise_equal(to_np(got[rows][:, cols]), to_np(want[rows][:, cols]), "other entries")
+
+
+@pytest.mark.parametrize("batch,rows,K", [(1, (1 << 25) + 70, 516), (3, (1 << 22) - 1, 8)])
+def test_more_rows_than_a_launch_counts(gpu, batch, rows, K):
+    """Rows whose work-items are 2^32 and more (35 GB of input and slices), and
+    batches cut between launches: the rows around the cuts as split alone."""
+    import ozaki_triton_amd as ozk
+    print(f"[rows] {batch}x{rows}x{K}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(K)
+    X = torch.randint(-100, 101, (batch, rows, K), generator=g, dtype=torch.int8, device=gpu)
+    sl, sc = ozk.split_matrix(X, 1, 7, torch.int8)
+    for b in {0, batch - 1}:
+        for at in {0, (1 << 23) - 2, (1 << 24) - 2, (1 << 25) - 2, rows - 4}:
+            if at + 4 <= rows:
+                wl, wc = ozk.split_matrix(X[b:b + 1, at:at + 4].contiguous(), 1, 7, torch.int8)
+                torch.cuda.synchronize()
+                assert torch.equal(sl[b:b + 1, :, at:at + 4], wl), (b, at)
+                assert torch.equal(sc[b:b + 1, :, at:at + 4], wc), (b, at)
+    del X, sl, sc
+    torch.cuda.empty_cache()
