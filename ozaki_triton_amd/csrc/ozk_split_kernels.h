@@ -128,9 +128,7 @@ template <typename ST, int MODE> struct Quant;
 template <> struct Quant<int8_t, kQF64> {
     OZK_DEV static uint32_t run(double x, const LevelScale &c, float *res) {
         const double q = x * c.inv64;
-        // |q| <= 2^7 (1 + 2^-18): the sum stays above -129, so truncation
-        // alone gives the reference's lower clamp
-        const int k = min(cvt_i32(q + __builtin_copysign(0.5, q)), 127);
+        const int k = max(min(cvt_i32(q + __builtin_copysign(0.5, q)), 127), -128);
         *res = (float)__builtin_fma(-(double)k, c.s64, x);
         return (uint32_t)k;
     }
@@ -138,7 +136,7 @@ template <> struct Quant<int8_t, kQF64> {
 template <> struct Quant<int8_t, kQExact> {
     OZK_DEV static uint32_t run(float r, const LevelScale &c, float *res) {
         const float q = __builtin_ldexpf(r, c.up);
-        const int k = min(cvt_i32(q + __builtin_copysignf(0x1.fffffep-2f, q)), 127);
+        const int k = max(min(cvt_i32(q + __builtin_copysignf(0x1.fffffep-2f, q)), 127), -128);
         *res = __builtin_fmaf(-(float)k, c.s, r);
         return (uint32_t)k;
     }
