@@ -199,7 +199,7 @@ static SplitParams converted_params(const SplitParams &p) {
 // 32 on gfx950, or all of a smaller partition.  Asked once per device; where
 // the runtime cannot say (no device: a workspace query on a host without a
 // GPU) MI355X's figure is assumed: 2 workgroups per CU (the kernels with
-// 169-205 VGPRs, one wave per SIMD each, fit twice in 512), so 64 per XCD
+// up to 175 VGPRs, one wave per SIMD each, fit twice in 512), so 64 per XCD
 // and at most 56 members (the row kernel's 64 chunks are cut to 56).
 // ---------------------------------------------------------------------------
 constexpr int kCusPerXcd = 32;
@@ -268,17 +268,18 @@ static SplitPlan plan_split_raw(const SplitParams &p, int x_dtype, int slice_dty
         if (rows_coop) return {kSplitRows, kRowsCoopVariant};
         if (rv >= 0) return {kSplitRows, rv};
     }
-    // columns of 64 KB and more: the cooperative kernel (the strip kernel's
-    // 16-byte row pieces cost more than the exchange from there on; measured
-    // over K = 1024..16384, N = 1024..8192, fp64 / fp32), and fp64 columns of
-    // 32 KB into 1 or 2 int8 slices when there are at least 2048 of them
-    // (alone, 0.90-0.94x the strip kernel's time at K = 4096, N = 2048..8192;
-    // 1.04x at N = 1024; fp16 slices gain nothing there, fp32 columns below
-    // 64 KB lose 1.1-1.3x).  With 3 or more slices the strip kernel and A's
-    // rows share one launch, and the whole call is faster that way: at K =
-    // 4096, 4 slices, 83.3 / 370.8 / 1163 us against 89.2 / 394.2 / 1197 for
-    // M x N = 128 x 2048, 1024 x 4096, 2048 x 8192, while 1 slice is 7-11%
-    // slower and 2 even.  A forced coop takes it for any length it holds
+    // columns of 64 KB and more: the cooperative kernel.  Alone against one
+    // workgroup's column groups, us, 2 int8 slices, 1024 / 2048 / 8192 columns:
+    // f64 K = 8192 27.6 (26.9) / 41.3 (48.4) / 154 (250), K = 16384 45.8 (51.5) /
+    // 108 (141) / 294 (542); f32 K = 16384 53.0 (34.6) / 81.4 (63.2) / 334 (382).
+    // Shorter columns lose: f64 K = 2048 22.5 (14.3) / 21.3 (14.6) / 37.6 (31.9),
+    // f32 K = 4096 21.4 (14.0) / 24.1 (15.8) / 59.6 (47.3), K = 8192 26.5 (20.0) /
+    // 43.9 (33.1) / 154 (176).  The line lies where it lay against column groups one
+    // 16-byte load wide, as does that of the 32 KB columns of fp64 into 1 or 2
+    // int8 slices, 2048 or more: even those are no longer faster this way (27.0
+    // against 22.2 at 2048 columns, 94.8 against 94.9 at 8192; the whole call, M x
+    // N = 1024 x 4096, 2 slices, 114 against 97).  A forced coop takes it for any
+    // length it holds
     const int64_t coop_max = coop_member_limit(kCoopMaxP);
     const bool coop_fits = cols_ok && coop_members(p.K, xsz, 8) <= coop_max;
     // columns too long for 32 chunks of 128-byte groups: 32-byte groups, whose
