@@ -94,6 +94,8 @@ ozk::SplitParams make_split_params(const void *X, int64_t batch, int64_t rows, i
     p.Kp = K;
     p.cols = 0;
     p.x_code = 0;
+    p.row_mul = 0;
+    p.row_shift = 0;
     p.resid = nullptr;
     p.fail_out = nullptr;
     return p;

@@ -47,6 +47,8 @@ struct SplitParams {
     int64_t Kp;    // elements a slice row is written to, K or more: zeros beyond K
     int cols;      // split_fused_kernel: the operand's columns, not its rows, are strided
     int x_code;    // ... and the dtype code of X
+    uint32_t row_mul;   // row / rows == (row * row_mul) >> 32 >> row_shift for row < 2^31
+    int row_shift;      // (row_mul 0: not given)
     float *resid;  // workspace: exchange words of the cooperative kernels, the
                    // transposed operand [batch, rows, K] (transpose + row path) or
                    // the fp32 copy of a narrow input

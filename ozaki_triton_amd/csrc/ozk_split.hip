@@ -442,6 +442,15 @@ static SplitParams fused_params(const SplitParams &p, const SplitPlan &plan, int
     SplitParams q = p;
     q.cols = plan.path == kSplitStrip;
     q.x_code = x_dtype;
+    q.row_mul = 0;
+    if (!q.cols && p.batch > 1 && p.rows > 1 && p.batch * p.rows < (int64_t)1 << 31) {
+        // the smallest s with rows <= 2^s; 2^(31+s) / rows rounded up is exact
+        // for every row below 2^31: row * (row_mul * rows - 2^(31+s)) < 2^(31+s)
+        int s = 0;
+        while (((int64_t)1 << s) < p.rows) ++s;
+        q.row_mul = (uint32_t)((((uint64_t)1 << (31 + s)) + (uint64_t)p.rows - 1) / (uint64_t)p.rows);
+        q.row_shift = s - 1;
+    }
     return q;
 }
 // Width of the column groups (SplitLaunch::fused): wide ones where they are

@@ -362,7 +362,9 @@ OZK_DEV void store_quad(void *base, int64_t off, bool there, uint32_t v[4]) {
 // ozaki_matmul, us, branches / one to a kernel: 192^3 f64 -> 4 int8 15.1 / 13.8,
 // 448^3 18.0 / 16.7, 16 x 512 x 128 x 512 f32 -> 3 fp16 30.8 / 30.1, 2688 x 448 x
 // 128 f32 -> 2 int8 15.8 / 14.1, 613 x 1492 x 1664 f32 -> 5 bf16 (triangle) 87.4 /
-// 83.9, 14 x 256 x 3724 x 158 f32 -> 3 int8 101.6 / 86.0.
+// 83.9, 14 x 256 x 3724 x 158 f32 -> 3 int8 101.6 / 86.0.  Whole rows beside columns
+// of any pitch keep their form (the split of 4 x 2240 rows and 111 columns of 1344,
+// f32 -> 3 bf16, 48.4 / 31.2; both any before).
 enum { kExact = 0, kWhole = 1, kAny = 2 };
 
 // The same value afresh: the row's limits, taken at each level through this,
@@ -432,6 +434,31 @@ OZK_DEV Quot quot(int64_t a, int64_t b) {
     return {a / b, a % b};
 }
 
+// Where row `row` (of all batches) starts in X, the slices and the scales.  Short
+// rows are bound by the scalar instructions before their first load (a wave of 4
+// to 8 elements a lane issues more of them than vector ones): one batch goes
+// without the division and half of the 64-bit products, several with a
+// multiplication for it.  With the operand's parameters no longer selected
+// from both operands' and the waves past a row's end idle, rows alone, f32 -> 2
+// fp16, us, before / now: 12000 of 192 8.8 / 6.8, 9000 of 704 13.4 / 9.1, 8960 of
+// 1280 22.6 / 16.6, 4 x 2240 of 1344 22.5 / 18.1; f64 -> 4 int8 11.6 / 9.6, 20.0 /
+// 16.6, 33.2 / 27.6, 34.4 / 29.3.
+struct RowAt {
+    int64_t x, slice, scale;
+};
+OZK_DEV RowAt row_at(const SplitParams &p, int64_t row) {
+    if (p.batch == 1) return {row * p.xs_r, row * p.ss_r, row * p.cs_r};
+    Quot at;
+    if (p.row_mul) {   // row < 2^31
+        at.q = __umulhi((uint32_t)row, p.row_mul) >> p.row_shift;
+        at.r = (uint32_t)row - (uint32_t)at.q * (uint32_t)p.rows;
+    } else {
+        at = quot(row, p.rows);
+    }
+    return {at.q * p.xs_b + at.r * p.xs_r, at.q * p.ss_b + at.r * p.ss_r,
+            at.q * p.cs_b + at.r * p.cs_r};
+}
+
 // ---------------------------------------------------------------------------
 // Row-resident split.  Block = RPB groups of G = 64*GW lanes; group g owns
 // global row block*RPB + g.  Lane t of a group holds elements
@@ -487,10 +514,11 @@ OZK_DEV void split_row(const SplitParams &p, int64_t xrow, int64_t srow, int K, 
         const int64_t sl = srow + l * p.ss_l;
         const int Ks = per_level_uniform(K), Kps = per_level_uniform(Kp);
         const int lt = per_level(t);
+        const int wt = __builtin_amdgcn_readfirstlane(lt);
 #pragma unroll
         for (int ch = 0; ch < NC; ++ch) {
             const int e0 = (ch * G + lt) * 4;
-            if (FORM != kExact && ch * G * 4 >= Kps) {   // a chunk past the row's end
+            if (FORM != kExact && (ch * G + wt) * 4 >= Kps) {   // the wave is past the row's end
                 if (decltype(first)::value)
 #pragma unroll
                     for (int u = 0; u < 4; ++u) w[ch * 4 + u] = 0.0f;
@@ -533,15 +561,13 @@ OZK_DEV void split_rows_body(const SplitParams &p, int64_t block, float (*red)[R
     const int64_t nrows = p.batch * p.rows;
     const int64_t grow = block * RPB + grp;
     const bool off = grow >= nrows;
-    const Quot at = quot(off ? 0 : grow, p.rows);
-    const int64_t b = at.q, r = at.r;
-    float *srow_scale = p.scales + b * p.cs_b + r * p.cs_r;
+    const RowAt at = row_at(p, off ? 0 : grow);
+    float *srow_scale = p.scales + at.scale;
     auto smax = [&](float m, int l) { return row_max<GW, RPB>(m, red, l & 1, grp, t); };
     auto put = [&](int l, const LevelScale &c) {
         if (!off && t == 0) srow_scale[l * p.cs_l] = c.s;
     };
-    const int64_t xrow = b * p.xs_b + r * p.xs_r, srow = b * p.ss_b + r * p.ss_r;
-    split_row<XC, ST, G, NC, FORM>(p, xrow, srow, (int)p.K, (int)p.Kp, off, t, smax, put);
+    split_row<XC, ST, G, NC, FORM>(p, at.x, at.slice, (int)p.K, (int)p.Kp, off, t, smax, put);
 }
 
 template <typename XC, typename ST, int GW, int RPB, int NC, int FORM>
@@ -672,11 +698,11 @@ OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, 
         put(l, c);
         const int64_t sl = sbase + l * p.ss_l;
         const int Ks = per_level(K), Kps = per_level(Kp), nc = per_level(ncol);
-        const int kpin = kin + 16;   // no padding from there on
+        const int kpw = __builtin_amdgcn_readfirstlane(Kps);   // of the wave's first row
 #pragma unroll
         for (int g = 0; g < NQ; ++g) {
             const int k0 = 4 * g * RPP;
-            if (SKIP && k0 >= kpin) {   // past the last row
+            if (SKIP && k0 >= kpw) {   // the wave is past the last row
                 if (decltype(first)::value)
 #pragma unroll
                     for (int dk = 0; dk < 4; ++dk)
@@ -684,27 +710,21 @@ OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, 
                         for (int u = 0; u < VEC; ++u) w[g][dk][u] = 0.0f;
                 continue;
             }
-            uint32_t qv[VEC][4];
+            // column by column: four slice values live at a time (all at once
+            // spilled scalar registers, and f32 into bf16 took 139 vector ones)
 #pragma unroll
-            for (int dk = 0; dk < 4; ++dk)
+            for (int u = 0; u < VEC; ++u) {
+                uint32_t qv[4];
 #pragma unroll
-                for (int u = 0; u < VEC; ++u)
-                    qv[u][dk] = Quant<ST, MODE>::run(src[g][dk][u], c[u], &w[g][dk][u]);
-            if (FORM == kExact || (FORM == kAny && col_ok && 4 * (g + 1) * RPP <= kin)) {
-#pragma unroll
-                for (int u = 0; u < VEC; ++u)
-                    Store4<ST>::run(p.slices, sl + u * p.ss_r + k0, qv[u]);
-            } else if (FORM == kWhole) {
-                if (k0 < Kps && nc > 0) {
-#pragma unroll
-                    for (int u = 0; u < VEC; ++u)
-                        store_quad<ST>(p.slices, sl + u * p.ss_r + k0, k0 < Ks, qv[u]);
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < VEC; ++u)
-                    if (u < nc)
-                        store_some<ST>(p.slices, sl + u * p.ss_r + k0, Ks - k0, Kps - k0, qv[u]);
+                for (int dk = 0; dk < 4; ++dk)
+                    qv[dk] = Quant<ST, MODE>::run(src[g][dk][u], c[u], &w[g][dk][u]);
+                const int64_t at = sl + u * p.ss_r + k0;
+                if (FORM == kExact || (FORM == kAny && col_ok && 4 * (g + 1) * RPP <= kin))
+                    Store4<ST>::run(p.slices, at, qv);
+                else if (FORM == kWhole) {
+                    if (k0 < Kps && nc > 0) store_quad<ST>(p.slices, at, k0 < Ks, qv);
+                } else if (u < nc)
+                    store_some<ST>(p.slices, at, Ks - k0, Kps - k0, qv);
             }
             // the residuals here, not at their first use (see split_row)
 #pragma unroll
@@ -767,30 +787,31 @@ __global__ __launch_bounds__(NT) void split_cols_kernel(SplitParams p) {
 // ---------------------------------------------------------------------------
 // One or both operands of a matmul in one launch (K <= 8192).  The first n0
 // workgroups split operand 0, the others operand 1; each operand is rows or
-// columns (SplitParams::cols).  Neither waits on another workgroup.
+// columns (SplitParams::cols), rows beside columns operand 1.  Neither waits on
+// another workgroup.  FORM: the rows' form, CFORM: the columns'.
 // ---------------------------------------------------------------------------
 struct FusedSplit {
     SplitParams op[2];
 };
-// (SEG = 0: rows only)
-template <typename XC, typename ST, int NT, int GW, int NC, int SEG, int NQ, int FORM>
-__global__ __launch_bounds__(NT) void split_fused_kernel(FusedSplit f, int64_t n0) {
-    const int which = (int64_t)blockIdx.x >= n0;
-    const SplitParams &p = f.op[which];
-    const int64_t g = (int64_t)blockIdx.x - (which ? n0 : 0);
+template <typename XC, typename ST, int NT, int GW, int NC, int SEG, int NQ, int FORM, int CFORM>
+__global__ __launch_bounds__(NT) void split_fused_kernel(FusedSplit f, uint32_t n0) {
+    const bool which = blockIdx.x >= n0;
+    const uint32_t g = blockIdx.x - (which ? n0 : 0);
     constexpr int RPB = NT / (64 * GW);
-    __shared__ union {
-        ColsShared<NT, (SEG > 0 ? SEG : 1), In<XC>::VEC> cols;
-        float rows[2][RPB][GW];
-    } sh;
     if constexpr (SEG > 0) {
-        if (p.cols) {
-            split_cols_body<XC, ST, NT, SEG, NQ, FORM>(
-                p, xcd_remap(g, which ? (int64_t)gridDim.x - n0 : n0), sh.cols);
-            return;
-        }
+        __shared__ union {
+            ColsShared<NT, SEG, In<XC>::VEC> cols;
+            float rows[2][RPB][GW];
+        } sh;
+        if (!which || f.op[1].cols)
+            split_cols_body<XC, ST, NT, SEG, NQ, CFORM>(
+                f.op[which], xcd_remap(g, which ? gridDim.x - n0 : n0), sh.cols);
+        else   // (not f.op[which]: every wave would load both and select)
+            split_rows_body<XC, ST, GW, RPB, NC, FORM>(f.op[1], g, sh.rows);
+    } else {
+        __shared__ float red[2][RPB][GW];
+        split_rows_body<XC, ST, GW, RPB, NC, FORM>(f.op[which], g, red);
     }
-    split_rows_body<XC, ST, GW, RPB, NC, FORM>(p, g, sh.rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -1275,6 +1296,8 @@ static hipError_t launch_long(const SplitParams &p, const SplitPlan &plan, hipSt
 //   K = 4096 <256,1,4>  N =  512 12.1 / 8.9 [14.6 / 10.0]
 //     wide   <512,2,4>  N = 2048 35.5 / 15.9   8192 118.8 / 79.5 [152.9 / 96.5]
 //   K = 8192 <512,1,4>  N = 2048 73.0 / 51.1 [97.5 / 58.4]
+// (<NT, SEG, NQ> here.)  Rows of up to 1024 take a wave each: two waves and their
+// exchange a level were 10.9 us against 9.1 for 9000 f32 rows of 704 alone.
 // Rows and columns in one launch, narrow / wide: 4096^2 f64 -> 5 int8 115 / 108,
 // 4096^2 f32 -> 2 fp16 68 / 66, f64 -> 4 int8 2048 rows and 4096 columns of
 // 2048 41.9 / 39.9, 4096 and 4096 of 1024 27.9 / 24.5 (two launches: 120,
@@ -1288,17 +1311,37 @@ static hipError_t launch_fused_cfg(const FusedSplit &f, int n, hipStream_t st) {
     auto blocks = [](const SplitParams &p) -> int64_t {
         return p.cols ? p.batch * ((p.rows + SW - 1) / SW) : (p.batch * p.rows + RPB - 1) / RPB;
     };
-    int form = kExact;
+    int form[2] = {kExact, kExact};   // rows, columns
+    bool has_rows = false;
     for (int i = 0; i < n; ++i) {
-        const int fi = split_form(f.op[i], f.op[i].cols, CAP, f.op[i].cols ? SW : RPB, VEC);
-        form = fi > form ? fi : form;
+        const int c = f.op[i].cols != 0;
+        const int fi = split_form(f.op[i], c, CAP, c ? SW : RPB, VEC);
+        form[c] = fi > form[c] ? fi : form[c];
+        has_rows |= !c;
     }
     const int64_t n0 = blocks(f.op[0]);
     const int64_t total = n0 + (n > 1 ? blocks(f.op[1]) : 0);
-    with_form(form, [&](auto fm) {
-        hipLaunchKernelGGL((split_fused_kernel<XC, ST, NT, GW, NC, SEG, NQ, decltype(fm)::value>),
-                           dim3((unsigned)total), dim3(NT), 0, st, f, n0);
-    });
+    // one form for both, but whole rows beside any columns (a ragged pitch of
+    // theirs) keep their own
+    const int all = form[0] > form[1] ? form[0] : form[1];
+    auto launch = [&](auto fm, auto cf) {
+        hipLaunchKernelGGL((split_fused_kernel<XC, ST, NT, GW, NC, SEG, NQ, decltype(fm)::value,
+                                               decltype(cf)::value>),
+                           dim3((unsigned)total), dim3(NT), 0, st, f, (uint32_t)n0);
+    };
+    if constexpr (SEG > 0) {
+        if (has_rows && form[0] != kAny && form[1] == kAny) {
+            launch(std::integral_constant<int, kWhole>{}, std::integral_constant<int, kAny>{});
+            return hipGetLastError();
+        }
+    } else if (n == 1) {
+        with_form(all, [&](auto fm) {
+            hipLaunchKernelGGL((split_rows_kernel<XC, ST, GW, RPB, NC, decltype(fm)::value>),
+                               dim3((unsigned)total), dim3(NT), 0, st, f.op[0]);
+        });
+        return hipGetLastError();
+    }
+    with_form(all, [&](auto fm) { launch(fm, fm); });
     return hipGetLastError();
 }
 template <typename XC, typename ST>
@@ -1310,8 +1353,8 @@ static hipError_t launch_fused_x(const FusedSplit &f, int n, int cls, int width,
     case 1: OZK_FUSED(256, 1, 1, 4, 1);
     case 3: OZK_FUSED(256, 1, 2, 0, 0);
     case 4: OZK_FUSED(256, 1, 2, 2, 1);
-    case 6: OZK_FUSED(256, 2, 2, 0, 0);
-    case 7: OZK_FUSED(256, 2, 2, 2, 2);
+    case 6: OZK_FUSED(256, 1, 4, 0, 0);
+    case 7: OZK_FUSED(256, 1, 4, 2, 2);
     case 9: OZK_FUSED(256, 4, 2, 0, 0);
     case 10: OZK_FUSED(256, 4, 2, 2, 4);
     case 12: OZK_FUSED(256, 4, 4, 0, 0);
@@ -1334,8 +1377,9 @@ template <typename ST>
 hipError_t SplitLaunch<ST>::fused(const SplitParams *p0, const SplitParams *p1, int cls, int width,
                                   int x_dtype, hipStream_t st) {
     FusedSplit f;
-    f.op[0] = *p0;
-    f.op[1] = p1 ? *p1 : *p0;
+    const bool swap = p1 && !p0->cols && p1->cols;   // columns first
+    f.op[0] = swap ? *p1 : *p0;
+    f.op[1] = p1 && !swap ? *p1 : *p0;
     const int n = p1 ? 2 : 1;
     if (x_dtype == 0) return launch_fused_x<double, ST>(f, n, cls, width, st);
     if (x_dtype == 1) return launch_fused_x<float, ST>(f, n, cls, width, st);

@@ -62,6 +62,49 @@ def test_whole_quads_infinite_entries(gpu, M, N, K, xdt, sdt):
     assert_bitwise_equal(to_np(got[rows][:, cols]), to_np(want[rows][:, cols]), "other entries")
 
 
+# batches of 1, 2, prime, a power of two and one more or less rows (the row's batch
+# is a multiplication), and workgroups of 1 and 4 rows that cross batches
+@pytest.mark.parametrize("batch,rows", [(1, 9), (9, 1), (5, 2), (6, 3), (3, 7), (4, 8), (3, 17), (2, 31),
+                                        (3, 127), (3, 257)])
+@pytest.mark.parametrize("K", [60, 192, 320, 703, 704, 1344, 2900])
+def test_batched_rows(oracle, gpu, batch, rows, K):
+    import ozaki_triton_amd as ozk
+    xdt, sdt = [(torch.float64, torch.int8), (torch.float32, torch.float16),
+                (torch.bfloat16, torch.int8)][(rows + K) % 3]
+    g = torch.Generator().manual_seed(batch * 1000 + rows)
+    X = torch.randn(batch, rows, K, generator=g, dtype=torch.float64).to(xdt)
+    alpha = ozk.compute_split_bits(K, sdt, torch.int32 if sdt == torch.int8 else torch.float32)
+    sl, sc = ozk.split_matrix(X.to(gpu), 2, alpha, sdt)
+    torch.cuda.synchronize()
+    osl, osc = oracle_split_batched(oracle, to_np(X), 2, alpha, sdt)
+    assert_bitwise_equal(to_np(sc), osc, "scales")
+    assert_bitwise_equal(to_np(sl), osl, "slices")
+
+
+# both splits in one launch: whole rows beside columns of any pitch, in every class
+# of K, and columns of A beside rows of B
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, True)])
+@pytest.mark.parametrize("xdt,sdt", [(torch.float64, torch.int8), (torch.float32, torch.int8),
+                                     (torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("batch,M,N,K", [(3, 5, 7, 96), (4, 33, 111, 320), (3, 130, 63, 704),
+                                         (2, 66, 97, 1344), (2, 34, 35, 2900), (1, 130, 111, 5600)])
+def test_whole_rows_beside_any_columns(gpu, batch, M, N, K, xdt, sdt, ta, tb):
+    import ozaki_triton_amd as ozk
+    g = torch.Generator().manual_seed(M * N + K)
+    A = torch.randn(batch, M, K, generator=g, dtype=torch.float64).to(xdt).to(gpu)
+    B = torch.randn(batch, K, N, generator=g, dtype=torch.float64).to(xdt).to(gpu)
+    A = A.mT.contiguous().mT if ta else A
+    B = B.mT.contiguous().mT if tb else B
+    got = ozk.ozaki_matmul(A, B, 3, sdt)
+    # each operand split alone, from contiguous rows (checked against the oracle above)
+    alpha = ozk.compute_split_bits(K, sdt, torch.int32 if sdt == torch.int8 else torch.float32)
+    a_sl, a_sc = ozk.split_matrix(A.contiguous(), 3, alpha, sdt)
+    b_sl, b_sc = ozk.split_matrix(B.mT.contiguous(), 3, alpha, sdt)
+    want = ozk.cross_gemm(a_sl, b_sl.transpose(-1, -2), a_sc, b_sc, 3, xdt)
+    torch.cuda.synchronize()
+    assert_bitwise_equal(to_np(got), to_np(want), f"{ta} {tb}")
+
+
 @pytest.mark.parametrize("batch,rows,K", [(1, (1 << 25) + 70, 516), (3, (1 << 22) - 1, 8)])
 def test_more_rows_than_a_launch_counts(gpu, batch, rows, K):
     """Rows whose work-items are 2^32 and more (35 GB of input and slices), and
