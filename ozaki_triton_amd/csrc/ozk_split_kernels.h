@@ -657,11 +657,15 @@ OZK_DEV void cols_scale(float m[VEC], ColsShared<NT, SEG, VEC> &sh, int buf, int
 // ncol: of its VEC columns, those that exist; col_ok, kin: uniform over the
 // workgroup, every lane has VEC columns / rows below kin exist for every lane.
 // FORM: kExact tests nothing; kWhole: every lane has all of its columns or none,
-// K and Kp are whole quads; SKIP: rows past the last one are left out.
+// K and Kp are whole quads; SKIP: rows past the last one are left out; BYCOL: a
+// column's four slice values are stored before the next column's are made.  With
+// all at once the kernels of K up to 8192 spilled scalar registers, and f32 into
+// bf16 took 139 vector ones; the cooperative ones take it, which by columns
+// grow past the 168 that leave three waves a SIMD.
 // scale(m, l, c): the level's constants of the lane's columns from its maxima;
 // put(l, c): stores their scales.
-template <typename XC, typename ST, int RPP, int NQ, int FORM, bool SKIP, typename Scale,
-          typename Put>
+template <typename XC, typename ST, int RPP, int NQ, int FORM, bool SKIP, bool BYCOL,
+          typename Scale, typename Put>
 OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, int Kp, int ncol,
                         bool col_ok, int kin, Scale &&scale, Put &&put) {
     using V = typename In<XC>::V;
@@ -698,7 +702,8 @@ OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, 
         put(l, c);
         const int64_t sl = sbase + l * p.ss_l;
         const int Ks = per_level(K), Kps = per_level(Kp), nc = per_level(ncol);
-        const int kpw = __builtin_amdgcn_readfirstlane(Kps);   // of the wave's first row
+        // of the wave's first row
+        const int kpw = SKIP ? __builtin_amdgcn_readfirstlane(Kps) : 0;
 #pragma unroll
         for (int g = 0; g < NQ; ++g) {
             const int k0 = 4 * g * RPP;
@@ -710,21 +715,39 @@ OZK_DEV void split_cols(const SplitParams &p, int64_t xb, int64_t sbase, int K, 
                         for (int u = 0; u < VEC; ++u) w[g][dk][u] = 0.0f;
                 continue;
             }
-            // column by column: four slice values live at a time (all at once
-            // spilled scalar registers, and f32 into bf16 took 139 vector ones)
+            if constexpr (BYCOL) {
 #pragma unroll
-            for (int u = 0; u < VEC; ++u) {
-                uint32_t qv[4];
+                for (int u = 0; u < VEC; ++u) {
+                    uint32_t qv[4];
+#pragma unroll
+                    for (int dk = 0; dk < 4; ++dk)
+                        qv[dk] = Quant<ST, MODE>::run(src[g][dk][u], c[u], &w[g][dk][u]);
+                    const int64_t at = sl + u * p.ss_r + k0;
+                    if (FORM == kExact || (FORM == kAny && col_ok && 4 * (g + 1) * RPP <= kin))
+                        Store4<ST>::run(p.slices, at, qv);
+                    else if (FORM == kWhole) {
+                        if (k0 < Kps && nc > 0) store_quad<ST>(p.slices, at, k0 < Ks, qv);
+                    } else if (u < nc)
+                        store_some<ST>(p.slices, at, Ks - k0, Kps - k0, qv);
+                }
+            } else {
+                static_assert(BYCOL || FORM != kWhole, "the cooperative kernels' forms");
+                uint32_t qv[VEC][4];
 #pragma unroll
                 for (int dk = 0; dk < 4; ++dk)
-                    qv[dk] = Quant<ST, MODE>::run(src[g][dk][u], c[u], &w[g][dk][u]);
-                const int64_t at = sl + u * p.ss_r + k0;
-                if (FORM == kExact || (FORM == kAny && col_ok && 4 * (g + 1) * RPP <= kin))
-                    Store4<ST>::run(p.slices, at, qv);
-                else if (FORM == kWhole) {
-                    if (k0 < Kps && nc > 0) store_quad<ST>(p.slices, at, k0 < Ks, qv);
-                } else if (u < nc)
-                    store_some<ST>(p.slices, at, Ks - k0, Kps - k0, qv);
+#pragma unroll
+                    for (int u = 0; u < VEC; ++u)
+                        qv[u][dk] = Quant<ST, MODE>::run(src[g][dk][u], c[u], &w[g][dk][u]);
+                if (FORM == kExact || (FORM == kAny && col_ok && 4 * (g + 1) * RPP <= kin)) {
+#pragma unroll
+                    for (int u = 0; u < VEC; ++u)
+                        Store4<ST>::run(p.slices, sl + u * p.ss_r + k0, qv[u]);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < VEC; ++u)
+                        if (u < nc)
+                            store_some<ST>(p.slices, sl + u * p.ss_r + k0, Ks - k0, Kps - k0, qv[u]);
+                }
             }
             // the residuals here, not at their first use (see split_row)
 #pragma unroll
@@ -774,7 +797,7 @@ OZK_DEV void split_cols_body(const SplitParams &p, int64_t sidx,
                 if (FORM == kExact || u < ncol) sc_base[l * p.cs_l + u * p.cs_r] = c[u].s;
         }
     };
-    split_cols<XC, ST, RPP, NQ, FORM, FORM != kExact>(
+    split_cols<XC, ST, RPP, NQ, FORM, FORM != kExact, true>(
         p, xb, sbase, (int)p.K - 4 * ro, (int)p.Kp - 4 * ro, ncol, col_ok, (int)p.K, scale, put);
 }
 
@@ -975,11 +998,16 @@ OZK_DEV void split_coop_body(const SplitParams &p, uint64_t *slot, int P, uint32
     };
     auto put = [](int, const LevelScale *) {};
     if (col_ok && kin == 4 * NG * RPP)
-        split_cols<XT, ST, RPP, NG, kExact, false>(p, xb, sbase, 0, 0, 0, true, 0, scale, put);
+        split_cols<XT, ST, RPP, NG, kExact, false, false>(p, xb, sbase, 0, 0, 0, true, 0, scale, put);
     else
-        split_cols<XT, ST, RPP, NG, kAny, false>(p, xb, sbase, K, Kp, ncol, col_ok, kin, scale, put);
+        split_cols<XT, ST, RPP, NG, kAny, false, false>(p, xb, sbase, K, Kp, ncol, col_ok, kin, scale,
+                                                        put);
 }
 
+// fp64 into int8, fp16 and fp32 slices takes 167 or 168 registers, three waves a
+// SIMD.  With one or two more, two waves, us: f64 2 x 8192^2 -> 4 int8
+// (split_pair_kernel) 338 -> 372, 4096 columns of 16384 -> 2 int8 176 -> 203, of
+// 8192 -> 3 fp16 121 -> 128.
 template <typename XT, typename ST, int RPL, int SEG>
 __global__ __launch_bounds__(kCoopNT) void split_coop_kernel(SplitParams p, uint64_t *slot, int P,
                                                              uint32_t want_tag,
