@@ -32,7 +32,7 @@
 //                         quotient; t = fl32(q +/- 0.5) as in the reference;
 //                         residual fma(-slice, s, x) = fl32(x - fl32(slice*s))
 //                         because slice*s is exact.
-//   fp16 slices: RN(q) from fp64 at level 0 of fp64 input (integer rounding);
+//   fp16 slices: RN(q) from fp64 at level 0 of fp64 input (f64_to_f16);
 //                elsewhere q is an fp32 value and the hardware RNE conversion
 //                rounds it once; slice*s is exact in fp32 in every case.
 //
@@ -52,8 +52,8 @@
 //                       K.  Either way the operand stays in VGPRs across the
 //                       levels: X is read from HBM once, each slice written
 //                       once.
-//   split_rows_kernel,  the same bodies for one operand of 8192 < K (rows of
-//   split_cols_kernel   up to 65536 elements, columns of up to 16384).
+//   split_rows_kernel   the same body for rows alone, of up to 65536 elements.
+//   split_cols_kernel   ... for columns alone, of 8192 < K <= 16384.
 //   split_rows_coop_kernel  rows longer than 16384: K chunks of a row in
 //                       separate workgroups that exchange the level maxima
 //                       through the workspace.

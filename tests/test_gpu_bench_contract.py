@@ -1,4 +1,4 @@
-"""bench.py's output line: the keys and meanings the driver reads.
+"""bench.py's output line: the keys and meanings its readers rely on.
 
 The GPU cases run bench.py in a child process at the reference's small
 configuration (C1, 256^3) and check its one JSON line; the CPU case checks
